@@ -126,7 +126,7 @@ struct RevStamp {
     double dt;           // time step of the bulk update
     int nseg, nact, every;
     size_t nel;
-    int launch[3][2];
+    int launch[3][2], planes;
     bool operator==(const RevStamp &o) const { return std::memcmp(this, &o, sizeof(RevStamp)) == 0; }
 };
 
@@ -198,6 +198,7 @@ RevStamp stamp_of(const Group *g, int every)
         st.launch[a][0] = g->launch[a].lds_blocks_per_cu;
         st.launch[a][1] = g->launch[a].ring;
     }
+    st.planes = g->planes ? 1 : 0;
     return st;
 }
 
@@ -236,6 +237,7 @@ int make_reverse(Group *g, Tape &tp)
     adj.cu_count = g->cu_count;
     for (int a = 0; a < 3; ++a)
         adj.launch[a] = g->launch[a];
+    adj.planes = g->planes;
     adj.doms.resize(1);
     Domain &ad = adj.doms[0];
     ad.nx = d.nx;
@@ -302,18 +304,15 @@ int backward_t(Group *g, const double *seed, double *grad_rho0, double *grad_t1,
             if (nseg > 0) {
                 hipLaunchKernelGGL(k_gather<T>, dim3(agrid), dim3(256), 0, g->stream, field(g->cur), d.seg_off, nseg,
                                    ns, d.nvox, rv.r0 + (size_t)j * nseg * ns);
-                if ((e = launch_agents(g)))
-                    return e;
             }
-            for (int axis = 0; axis < 3; ++axis)
-                if ((e = launch_sweep(g, axis)))
-                    return e;
+            if ((e = launch_step(g, nseg > 0)))
+                return e;
         }
         for (int j = L - 1; j >= 0; --j) {
             hipLaunchKernelGGL(k_zero_zfaces<T>, dim3(zgrid), dim3(256), 0, g->stream,
                                static_cast<T *>(ad.field[adj.cur]), d.d_dact, d.nx, d.ny, d.nz, ns);
             int e;
-            if ((e = launch_sweep(&adj, 2)) || (e = launch_sweep(&adj, 1)) || (e = launch_sweep(&adj, 0)))
+            if ((e = launch_step_adjoint(&adj)))
                 return set_error(g, e, adj.err);
             if (nseg > 0)
                 hipLaunchKernelGGL(k_agents_adjoint<T>, dim3(agrid), dim3(256), 0, g->stream,
@@ -362,7 +361,7 @@ int backward_t(Group *g, const double *seed, double *grad_rho0, double *grad_t1,
             if ((rc = hip_check(g, hipGraphLaunch(it->second, g->stream), "adjoint graph launch")))
                 return rc;
         }
-        // three buffer swaps per step on both sides
+        // one or three buffer swaps per step on both sides
         g->cur = tp.start ^ (L & 1);
         adj.cur = a0 ^ (L & 1);
     }

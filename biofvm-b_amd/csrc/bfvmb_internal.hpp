@@ -23,12 +23,29 @@
 namespace bfvmb {
 
 constexpr int kWave = 64;
+constexpr size_t kLdsBytes = 160 * 1024;  // LDS of one CU
+
+// Per-phase prefix sums over the domains of a group (work items of a launch).  Planes that are
+// swept whole in LDS (resident.hip) come in size classes by the LDS a workgroup takes, one launch
+// each, so that small members of a batch do not run at the occupancy of large ones; the domains
+// whose planes do not fit ("rest") are swept by the kernels of lod.hip.
+constexpr int kClasses = 5;  // up to 20, 40, 80 and 160 KB, and 160 KB in the denser layout
+enum Phase {
+    kAgents0 = 0,                     // agent work items
+    kSweep0 = 1,                      // x, y, z tiles
+    kBulk0 = 4,                       // bulk elements
+    kPlane0 = 5,                      // planes in LDS, by class
+    kRest0 = kPlane0 + kClasses,      // agents, x, y tiles of the domains outside those
+    kPhases = kRest0 + 3
+};
 
 // Per-axis Thomas tables, FP64 on both storage paths, [nsub][n].
 struct AxisTables {
     const double *den;   // denominators  (thomas_denom{x,y,z})
     const double *cc;    // upper factors (thomas_c{x,y,z})
     const double *rden;  // RN(1/den)
+    const double *rlow;  // low part of 1/den: fma(a, rden, a*rlow) is RN(a/den) (reciprocal_pair)
+    const double *nopair;  // [nsub] number of rows without such a pair
 };
 
 // Device descriptor of one domain (plain data, copied to the GPU).
@@ -46,6 +63,7 @@ struct DomainDesc {
     const double *t1, *t2;       // agents: [nsub][nact] temp1 / temp2, sorted order
     const int *xseg;             // agents: [x-sweep tiles per substrate + 1] first segment of
                                  // each tile of 64 rows (z*ny + y), or nullptr: no agents
+    const int *zseg;             // agents: [nz + 1] first segment of each z plane, or nullptr: no agents
     const double *bulk_ts;       // bulk: [nsub][nz][ny][nx] target*supply (nullptr: none)
     const double *bulk_us;       // bulk: [nsub][nz][ny][nx] uptake+supply
     double dt;                   // time step frozen by set_coefficients
@@ -87,7 +105,7 @@ struct Domain {
     double dx = 0.0;
     size_t nvox = 0;
     void *field[2] = {nullptr, nullptr};
-    double *coef = nullptr;  // c1[nsub] | per axis den, cc, rden [nsub][n]
+    double *coef = nullptr;  // c1[nsub] | per axis den, cc, rden, rlow [nsub][n], nopair [nsub]
     bool have_coef = false;
     double dt = 0.0;
     std::vector<double> D, decay;
@@ -104,6 +122,8 @@ struct Domain {
     double *t1 = nullptr, *t2 = nullptr;
     size_t seg_cap = 0, act_cap = 0;  // segments / agents the device arrays have room for
     int *xseg = nullptr;           // first segment of each x-sweep tile (rebuilt with the descriptors)
+    int *zseg = nullptr;           // first segment of each z plane (likewise)
+    int plane_class = -1;          // LDS size class of its z planes, -1: they do not fit
     std::vector<int> agent_order;  // sorted position -> index in the caller's agent list (after
                                    // moves: current once domain_agent_order has run)
     std::vector<long long> agent_off;  // device offset of each sorted agent's voxel, as set
@@ -116,7 +136,7 @@ struct Domain {
 
 // Offsets inside a domain's coefficient block, in doubles.
 struct CoefLayout {
-    size_t c1, den[3], cc[3], rden[3], total;
+    size_t c1, den[3], cc[3], rden[3], rlow[3], nopair[3], total;
 };
 CoefLayout coef_layout(const Domain &d);
 
@@ -131,11 +151,13 @@ struct Group {
     LaunchShape launch[3];
     size_t max_lds_per_block = 0;
     int cu_count = 0;
-    // device descriptors and per-phase prefix sums (0 = agent work items, 1..3 = x,y,z
-    // tiles, 4 = bulk elements)
+    // x and y sweeps on planes in LDS where they fit; off where a launch shape was asked for, or the
+    // autotuner found the separate sweeps faster
+    bool planes = true;
+    // device descriptors and per-phase prefix sums (Phase)
     void *d_desc = nullptr;
     long long *d_prefix = nullptr;
-    std::vector<long long> prefix[5];
+    std::vector<long long> prefix[kPhases];
     bool desc_dirty = true;
     // FP64 steps apply the cell sources and sinks inside the x sweep's launch when no x-sweep
     // tile holds more than kFuseMaxSegsPerTile occupied voxels (set with the descriptors)
@@ -152,8 +174,12 @@ struct Group {
 };
 
 // Launchers (lod.hip, field.hip): one kernel over all domains of the group.
-int launch_sweep(Group *g, int axis);   // field[cur] -> field[cur^1] for every domain
-int launch_sweep_x_agents(Group *g);    // cell sources/sinks, then the x sweep, in one launch
+// field[cur] -> field[cur^1] for every domain, or for those not swept in LDS (rest)
+int launch_sweep(Group *g, int axis, bool rest = false);
+int launch_planes(Group *g, bool yx, bool agents);  // resident planes, in place on field[cur]
+void resident_class(const Group *g, Domain &d);
+int resident_lds_attributes(size_t bytes);
+int launch_sweep_x_agents(Group *g, bool rest = false);  // cell sources/sinks, then the x sweep, in one launch
 int launch_xseg(Group *g, const Domain &d);  // xseg from the domain's segment list
 // Occupied voxels per x-sweep tile above which the agent update runs as its own kernel: the
 // fused update is one wavefront per tile working through its segments 256 at a time, so a
@@ -163,7 +189,7 @@ int launch_xseg(Group *g, const Domain &d);  // xseg from the domain's segment l
 // (3788) 3.398 against 3.389; 5M (5785) 3.573 against 3.430.  640^3 x 8 with 10M agents
 // (4639): fused x sweep 12.30 ms against 9.72 + 2.26 separate.
 constexpr int kFuseMaxSegsPerTile = 3072;
-int launch_agents(Group *g);            // in place on field[cur]
+int launch_agents(Group *g, bool rest = false);  // in place on field[cur]
 int launch_bulk(Group *g, double dt);   // in place on field[cur], domains with bulk rates;
                                         // dt <= 0: each domain's own time step
 int launch_aos_to_soa(Group *g, Domain &d, const double *d_aos, void *d_soa);
@@ -177,6 +203,7 @@ void lod_constants(int nsub, const double *D, const double *decay, double dt, do
                    double *c1, double *c2, double *c3, double *c3a);
 void thomas_axis(int n, int nsub, const double *c1, const double *c2, const double *c3,
                  const double *c3a, double *den, double *cc);
+bool reciprocal_pair(double d, double *hi, double *lo);
 
 // Group operations behind both ABIs (group.hip).
 int set_error(Group *g, int code, const std::string &msg);
@@ -210,6 +237,8 @@ int domain_download_device(Group *g, int i, double *d_rho);
 void free_remap(Domain &d);
 void free_agents(Domain &d);  // group.hip: releases a domain's agent list (and its remap state)
 int group_bulk(Group *g, double dt);
+int launch_step(Group *g, bool with_agents);  // one step without the bulk update
+int launch_step_adjoint(Group *g);            // its transposed sweeps, Dirichlet value 0, z first
 int group_steps(Group *g, int nsteps, bool with_agents, bool use_graph);
 int group_set_stream(Group *g, void *stream);
 int group_launch_phase(Group *g, int phase, int count);

@@ -50,16 +50,16 @@ __global__ __launch_bounds__(256) void k_agents(const DomainDesc<T> *__restrict_
     *p = (T)r;
 }
 
-// First segment of each x-sweep tile (64 consecutive rows r = z*ny + y of a substrate): the
-// smallest k with seg_off[k] >= 64 * t * nx, t = 0 .. ntiles (t = ntiles: nseg).  The list is
+// First segment of each tile of `unit` consecutive rows r = z*ny + y of a substrate (x-sweep tiles:
+// 64, z planes: ny): the smallest k with seg_off[k] >= unit * t * nx, t = 0 .. ntiles (the last: nseg).  The list is
 // sorted by voxel, so a tile's occupied voxels are the segments [xseg[t], xseg[t + 1]).
 __global__ __launch_bounds__(256) void k_xseg(const long long *__restrict__ seg_off, int nseg, int nx,
-                                              long long nrows, int ntiles, int *__restrict__ xseg)
+                                              long long nrows, int unit, int ntiles, int *__restrict__ xseg)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t > ntiles)
         return;
-    const long long v = min((long long)t * kWave, nrows) * nx;
+    const long long v = min((long long)t * unit, nrows) * nx;
     int lo = 0, hi = nseg;  // first k in [lo, hi] with seg_off[k] >= v
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
@@ -165,18 +165,19 @@ __global__ __launch_bounds__(256) void k_densities_at(const T *__restrict__ f, i
 }
 
 template <class T>
-int launch_agents_t(Group *g)
+int launch_agents_t(Group *g, bool rest)
 {
     int rc = sync_descriptors(g);
     if (rc)
         return rc;
     const int ndom = (int)g->doms.size();
-    const long long work = g->prefix[0][ndom];
+    const int phase = rest ? kRest0 : kAgents0;
+    const long long work = g->prefix[phase][ndom];
     if (work == 0)
         return BFVMB_OK;
     const unsigned grid = (unsigned)((work + 255) / 256);
     hipLaunchKernelGGL(k_agents<T>, dim3(grid), dim3(256), 0, g->stream, static_cast<const DomainDesc<T> *>(g->d_desc),
-                       g->d_prefix, ndom, g->cur);
+                       g->d_prefix + (size_t)phase * (ndom + 1), ndom, g->cur);
     return hip_check(g, hipGetLastError(), "agents launch");
 }
 
@@ -313,15 +314,17 @@ int launch_xseg(Group *g, const Domain &d)
     const long long nrows = (long long)d.ny * d.nz;
     const int ntiles = (int)((nrows + kWave - 1) / kWave);
     hipLaunchKernelGGL(k_xseg, dim3((unsigned)((ntiles + 1 + 255) / 256)), dim3(256), 0, g->stream, d.seg_off, d.nseg,
-                       d.nx, nrows, ntiles, d.xseg);
+                       d.nx, nrows, kWave, ntiles, d.xseg);
+    hipLaunchKernelGGL(k_xseg, dim3((unsigned)((d.nz + 1 + 255) / 256)), dim3(256), 0, g->stream, d.seg_off, d.nseg,
+                       d.nx, nrows, d.ny, d.nz, d.zseg);
     return hip_check(g, hipGetLastError(), "agent tile index launch");
 }
 
-int launch_agents(Group *g)
+int launch_agents(Group *g, bool rest)
 {
     if (g->precision == BFVMB_FP64)
-        return launch_agents_t<double>(g);
-    return launch_agents_t<float>(g);
+        return launch_agents_t<double>(g, rest);
+    return launch_agents_t<float>(g, rest);
 }
 
 int launch_aos_to_soa_f64(Group *g, Domain &d, const double *d_aos, double *d_soa)
@@ -337,11 +340,11 @@ int launch_bulk(Group *g, double dt)
     if (rc)
         return rc;
     const int ndom = (int)g->doms.size();
-    const long long work = g->prefix[4][ndom];
+    const long long work = g->prefix[kBulk0][ndom];
     if (work == 0)
         return BFVMB_OK;
     const unsigned grid = (unsigned)((work + 255) / 256);
-    const long long *pre = g->d_prefix + (size_t)4 * (ndom + 1);
+    const long long *pre = g->d_prefix + (size_t)kBulk0 * (ndom + 1);
     if (g->precision == BFVMB_FP64)
         hipLaunchKernelGGL(k_bulk<double>, dim3(grid), dim3(256), 0, g->stream,
                            static_cast<const DomainDesc<double> *>(g->d_desc), pre, ndom, g->cur, dt);

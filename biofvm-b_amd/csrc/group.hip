@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <unordered_map>
 
 #include "bfvmb_internal.hpp"
 
@@ -38,8 +39,12 @@ CoefLayout coef_layout(const Domain &d)
         off += s * n[a];
         L.rden[a] = off;
         off += s * n[a];
+        L.rlow[a] = off;
+        off += s * n[a];
+        L.nopair[a] = off;
+        off += s;
     }
-    L.total = off;
+    L.total = off + 16;  // scalar loads read a batch of entries at a time
     return L;
 }
 
@@ -89,7 +94,8 @@ std::vector<DomainDesc<T>> build_descs(Group *g)
             const CoefLayout L = coef_layout(d);
             e.c1 = d.coef + L.c1;
             for (int a = 0; a < 3; ++a)
-                e.tab[a] = AxisTables{d.coef + L.den[a], d.coef + L.cc[a], d.coef + L.rden[a]};
+                e.tab[a] = AxisTables{d.coef + L.den[a], d.coef + L.cc[a], d.coef + L.rden[a], d.coef + L.rlow[a],
+                                      d.coef + L.nopair[a]};
         }
         e.dval = static_cast<const T *>(d.d_dval);
         e.dact = d.d_dact;
@@ -99,6 +105,7 @@ std::vector<DomainDesc<T>> build_descs(Group *g)
         e.t1 = d.t1;
         e.t2 = d.t2;
         e.xseg = d.nseg > 0 ? d.xseg : nullptr;
+        e.zseg = d.nseg > 0 ? d.zseg : nullptr;
         e.bulk_ts = d.bulk;
         e.bulk_us = d.bulk ? d.bulk + d.nvox * d.nsub : nullptr;
         e.dt = d.dt;
@@ -133,21 +140,29 @@ int sync_descriptors(Group *g)
     if (!g->desc_dirty)
         return BFVMB_OK;
     const size_t nd = g->doms.size();
-    for (int p = 0; p < 5; ++p)
+    for (int p = 0; p < kPhases; ++p)
         g->prefix[p].assign(nd + 1, 0);
     for (size_t i = 0; i < nd; ++i) {
-        const Domain &d = g->doms[i];
-        const long long tx = (long long)((d.ny * (long long)d.nz + kWave - 1) / kWave) * d.nsub;
-        const long long ty = (long long)((d.nx * (long long)d.nz + kWave - 1) / kWave) * d.nsub;
-        const long long tz = (long long)((d.nx * (long long)d.ny + kWave - 1) / kWave) * d.nsub;
-        g->prefix[0][i + 1] = g->prefix[0][i] + (long long)d.nseg * d.nsub;
-        g->prefix[1][i + 1] = g->prefix[1][i] + tx;
-        g->prefix[2][i + 1] = g->prefix[2][i] + ty;
-        g->prefix[3][i + 1] = g->prefix[3][i] + tz;
-        g->prefix[4][i + 1] = g->prefix[4][i] + (d.bulk ? (long long)d.nvox * d.nsub : 0);
+        Domain &d = g->doms[i];
+        resident_class(g, d);
+        if (d.plane_class >= 0 && g->prefix[kPlane0 + d.plane_class][i] + (long long)d.nz * d.nsub > (1 << 30))
+            d.plane_class = -1;  // a launch counts its planes in int
+        long long work[kPhases] = {};
+        work[kAgents0] = (long long)d.nseg * d.nsub;
+        work[kSweep0] = (long long)((d.ny * (long long)d.nz + kWave - 1) / kWave) * d.nsub;
+        work[kSweep0 + 1] = (long long)((d.nx * (long long)d.nz + kWave - 1) / kWave) * d.nsub;
+        work[kSweep0 + 2] = (long long)((d.nx * (long long)d.ny + kWave - 1) / kWave) * d.nsub;
+        work[kBulk0] = d.bulk ? (long long)d.nvox * d.nsub : 0;
+        if (d.plane_class >= 0)
+            work[kPlane0 + d.plane_class] = (long long)d.nz * d.nsub;
+        else
+            for (int p = 0; p < 3; ++p)
+                work[kRest0 + p] = work[p];
+        for (int p = 0; p < kPhases; ++p)
+            g->prefix[p][i + 1] = g->prefix[p][i] + work[p];
     }
     std::vector<long long> flat;
-    for (int p = 0; p < 5; ++p)
+    for (int p = 0; p < kPhases; ++p)
         flat.insert(flat.end(), g->prefix[p].begin(), g->prefix[p].end());
     int rc;
     const size_t desc_bytes = nd * (g->precision == BFVMB_FP64 ? sizeof(DomainDesc<double>) : sizeof(DomainDesc<float>));
@@ -225,6 +240,7 @@ int group_init(Group *g, int ndom, const int *nx, const int *ny, const int *nz, 
         return rc;
     g->stream = g->own_stream;
     if ((rc = hip_check(g, (hipError_t)sweep_lds_attributes(g->max_lds_per_block), "LDS attributes")) ||
+        (rc = hip_check(g, (hipError_t)resident_lds_attributes(g->max_lds_per_block), "LDS attributes")) ||
         (rc = scratch_setup(g)))
         return rc;
     g->doms.resize(ndom);
@@ -245,6 +261,7 @@ int group_init(Group *g, int ndom, const int *nx, const int *ny, const int *nz, 
             (rc = hip_check(g, hipMalloc((void **)&d.d_dact, d.nsub), "dirichlet flags")) ||
             (rc = hip_check(g, hipMalloc((void **)&d.xseg, ((d.ny * (size_t)d.nz + kWave - 1) / kWave + 1) * sizeof(int)),
                             "agent tile index")) ||
+            (rc = hip_check(g, hipMalloc((void **)&d.zseg, (d.nz + 1) * sizeof(int)), "agent plane index")) ||
             (rc = hip_check(g, hipMemsetAsync(d.field[0], 0, bytes, g->stream), "zero field")) ||
             (rc = upload_dirichlet(g, d)))
             return rc;
@@ -269,6 +286,7 @@ void group_free(Group *g)
         (void)hipFree(d.d_dval);
         (void)hipFree(d.d_dact);
         (void)hipFree(d.xseg);
+        (void)hipFree(d.zseg);
         (void)hipFree(d.d_dface);
     }
     adjoint_free(g);
@@ -309,6 +327,8 @@ int domain_set_coefficients(Group *g, int i, const double *D, const double *deca
     std::vector<double> blob(L.total);
     for (int s = 0; s < ns; ++s)
         blob[L.c1 + s] = c1[s];
+    // the recursion settles, and the axes share it up to their last row: few distinct values
+    std::unordered_map<double, double> pairs;
     for (int a = 0; a < 3; ++a) {
         std::vector<double> den((size_t)ns * n[a]), cc((size_t)ns * n[a]);
         thomas_axis(n[a], ns, c1.data(), c2.data(), c3.data(), c3a.data(), den.data(), cc.data());
@@ -316,6 +336,16 @@ int domain_set_coefficients(Group *g, int i, const double *D, const double *deca
             blob[L.den[a] + k] = den[k];
             blob[L.cc[a] + k] = cc[k];
             blob[L.rden[a] + k] = 1.0 / den[k];
+            if (g->elem == 4)  // FP32 storage multiplies by RN(1/den)
+                continue;
+            auto it = pairs.find(den[k]);
+            if (it == pairs.end()) {
+                double hi, lo;
+                it = pairs.emplace(den[k], reciprocal_pair(den[k], &hi, &lo) ? lo : std::nan("")).first;
+            }
+            blob[L.rlow[a] + k] = it->second;
+            if (std::isnan(it->second))
+                blob[L.nopair[a] + k / n[a]] += 1.0;
         }
     }
     const size_t bytes = blob.size() * sizeof(double);
@@ -633,32 +663,58 @@ int group_bulk(Group *g, double dt)
 }
 
 // The step's cell sources and sinks and its x sweep: one launch (fuse_agents) or two.
-static int launch_agents_and_x(Group *g)
+static int launch_agents_and_x(Group *g, bool rest = false)
 {
     if (g->fuse_agents)
-        return launch_sweep_x_agents(g);
-    int rc = launch_agents(g);
-    return rc ? rc : launch_sweep(g, 0);
+        return launch_sweep_x_agents(g, rest);
+    int rc = launch_agents(g, rest);
+    return rc ? rc : launch_sweep(g, 0, rest);
+}
+
+int launch_step(Group *g, bool with_agents)
+{
+    int rc;
+    // planes in LDS, with their cell sources and sinks, in place; then the domains whose planes
+    // do not fit, through the other buffer and back
+    const bool rest = g->planes;
+    if (rest && (rc = launch_planes(g, false, with_agents)))
+        return rc;
+    // FP64: the cell sources and sinks run inside the x sweep, tile by tile, before it
+    // reads each tile (results identical to a separate pass; one launch fewer), unless a
+    // tile is dense (kFuseMaxSegsPerTile).  FP32 keeps the separate pass: its x sweep runs
+    // one wavefront per SIMD, which leaves no other wavefront to cover the update's latency.
+    if ((!rest || g->prefix[kRest0 + 1].back() > 0) &&
+        ((rc = with_agents ? launch_agents_and_x(g, rest) : launch_sweep(g, 0, rest)) ||
+         (rc = launch_sweep(g, 1, rest))))
+        return rc;
+    return launch_sweep(g, 2);
+}
+
+int launch_step_adjoint(Group *g)
+{
+    int rc = launch_sweep(g, 2);
+    if (rc)
+        return rc;
+    const bool rest = g->planes;
+    if (rest && (rc = launch_planes(g, true, false)))
+        return rc;
+    if (!rest || g->prefix[kRest0 + 1].back() > 0)
+        if ((rc = launch_sweep(g, 1, rest)) || (rc = launch_sweep(g, 0, rest)))
+            return rc;
+    return BFVMB_OK;
 }
 
 static int eager_steps(Group *g, int nsteps, bool with_agents)
 {
-    const bool bulk = g->prefix[4].back() > 0;
+    const bool bulk = g->prefix[kBulk0].back() > 0;
     for (int s = 0; s < nsteps; ++s) {
         int rc;
         // time loop of a step: bulk sources/sinks, cell sources/sinks, LOD
         // (BioFVM_microenvironment.cpp:1110-1169, BioFVM_parallel.cpp:693-1395)
         if (with_agents && bulk && (rc = launch_bulk(g, 0.0)))
             return rc;
-        // FP64: the cell sources and sinks run inside the x sweep, tile by tile, before it
-        // reads each tile (results identical to a separate pass; one launch fewer), unless a
-        // tile is dense (kFuseMaxSegsPerTile).  FP32 keeps the separate pass: its x sweep runs
-        // one wavefront per SIMD, which leaves no other wavefront to cover the update's latency.
-        if ((rc = with_agents ? launch_agents_and_x(g) : launch_sweep(g, 0)))
+        if ((rc = launch_step(g, with_agents)))
             return rc;
-        for (int axis = 1; axis < 3; ++axis)
-            if ((rc = launch_sweep(g, axis)))
-                return rc;
     }
     return BFVMB_OK;
 }
@@ -700,7 +756,7 @@ int group_steps(Group *g, int nsteps, bool with_agents, bool use_graph)
     }
     if ((rc = hip_check(g, hipGraphLaunch(it->second, g->stream), "graph launch")))
         return rc;
-    g->cur = start ^ (nsteps & 1);  // three buffer swaps per step
+    g->cur = start ^ (nsteps & 1);  // one or three buffer swaps per step
     return BFVMB_OK;
 }
 
@@ -731,6 +787,9 @@ int group_set_launch(Group *g, int sweep, long long grid, int bpc, int ring)
             g->launch[a].lds_blocks_per_cu = bpc;
             g->launch[a].ring = ring;
         }
+    // a shape asked for is a shape of the separate sweeps
+    auto shaped = [&](int a) { return g->launch[a].grid || g->launch[a].lds_blocks_per_cu || g->launch[a].ring; };
+    g->planes = !shaped(0) && !shaped(1);
     clear_graphs(g);
     return BFVMB_OK;
 }
@@ -764,8 +823,9 @@ int group_autotune(Group *g, int reps, int *chosen)
         rc = hip_check(g, hipEventCreate(&e0), "event");
     if (!rc)
         rc = hip_check(g, hipEventCreate(&e1), "event");
+    float best_ms[3] = {1e30f, 1e30f, 1e30f};
     for (int axis = 0; axis < 3 && !rc; ++axis) {
-        float best = 1e30f;
+        float &best = best_ms[axis];
         LaunchShape best_shape;
         // y/z: rows in flight; x: the FP32 variant by its chunks in flight (FP64 has one)
         const int yz_rings[2] = {32, 64}, x_rings[4] = {1, 2, 3, 4};
@@ -804,6 +864,31 @@ int group_autotune(Group *g, int reps, int *chosen)
             chosen[3 * axis + 2] = (int)(best * 1000.f / reps);  // microseconds per launch
         }
     }
+    // planes in LDS (both sweeps) against the separate sweeps at those shapes
+    const bool planes = g->planes;
+    bool any = false;
+    for (const Domain &d : g->doms)
+        any = any || d.plane_class >= 0;
+    auto once = [&]() -> int {
+        int e = launch_planes(g, false, false);
+        if (!e && g->prefix[kRest0 + 1].back() > 0 && !(e = launch_sweep(g, 0, true)))
+            e = launch_sweep(g, 1, true);
+        return e;
+    };
+    g->planes = true;
+    float ms = 0.f;
+    if (any && !rc && !(rc = once())) {
+        (void)hipEventRecord(e0, g->stream);
+        for (int k = 0; k < reps && !rc; ++k)
+            rc = once();
+        (void)hipEventRecord(e1, g->stream);
+        if (!rc)
+            rc = hip_check(g, hipEventSynchronize(e1), "autotune timing");
+        if (!rc && hipEventElapsedTime(&ms, e0, e1) == hipSuccess)
+            g->planes = ms < best_ms[0] + best_ms[1];
+    }
+    if (rc)
+        g->planes = planes;
     if (e0)
         (void)hipEventDestroy(e0);
     if (e1)

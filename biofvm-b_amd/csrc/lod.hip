@@ -1051,8 +1051,6 @@ __global__ __launch_bounds__(64, (x_waves_per_simd<T, REGC>())) void k_sweep_x(c
     }
 }
 
-constexpr size_t kLdsBytes = 160 * 1024;
-
 struct Shape {
     long long grid;  // 0 = one block per tile
     int bpc;         // sweep wavefronts sharing one CU's LDS
@@ -1192,19 +1190,21 @@ hipError_t x_attributes(int bytes)
 }
 
 template <class T>
-int launch_sweep_t(Group *g, int axis, bool agents)
+int launch_sweep_t(Group *g, int axis, bool agents, bool rest)
 {
     int rc = sync_descriptors(g);
     if (rc)
         return rc;
     const int ndom = (int)g->doms.size();
+    // rest: only the domains whose planes are not swept in LDS
+    auto skip = [&](const Domain &d) { return rest && d.plane_class >= 0; };
     const Shape sh = shape_of(g, axis);
     XVariant xv = x_variant<T>(sh.bpc, axis == 0 ? sh.ring : 0);
     if (axis == 0 && xv.tl) {
         // tables in LDS only where every domain's tables fit beside the smallest line store
         constexpr int W = x_chunk<T>();
         for (const Domain &d : g->doms)
-            if (16 * (size_t)d.nx + (size_t)kWave * (W + 1) * sizeof(T) +
+            if (!skip(d) && 16 * (size_t)d.nx + (size_t)kWave * (W + 1) * sizeof(T) +
                     (size_t)kWave * ((size_t)xv.pc * W + 1) * sizeof(T) > g->max_lds_per_block)
                 xv.tl = false;
     }
@@ -1214,6 +1214,8 @@ int launch_sweep_t(Group *g, int axis, bool agents)
     // one 16-column chunk
     size_t need = 0;
     for (const Domain &d : g->doms) {
+        if (skip(d))
+            continue;
         size_t full, floor;
         if (axis == 0) {
             constexpr int W = x_chunk<T>();
@@ -1238,6 +1240,8 @@ int launch_sweep_t(Group *g, int axis, bool agents)
     if (axis == 0) {
         constexpr int W = x_chunk<T>();
         for (const Domain &d : g->doms) {
+            if (skip(d))
+                continue;
             const int L = x_line_store<T>(d.nx, (long long)lds, xv.tl);
             if (L < W || (xv.regc > 0 && (d.nx + W - 1) / W > L / W && L / W < xv.pc))
                 return set_error(g, BFVMB_ERR_ARG, "sweep: LDS budget too small for the x line store");
@@ -1248,6 +1252,8 @@ int launch_sweep_t(Group *g, int axis, bool agents)
         // that fits every such domain
         int minL = 1 << 30;
         for (const Domain &d : g->doms) {
+            if (skip(d))
+                continue;
             const int n = axis == 1 ? d.ny : d.nz;
             const int L = yz_line_store<T>(n, (long long)lds, axis == 1 ? yz_scalar<T, 1>(g) : yz_scalar<T, 2>(g));
             if (L < n)
@@ -1259,8 +1265,9 @@ int launch_sweep_t(Group *g, int axis, bool agents)
         if (minL < ring)
             return set_error(g, BFVMB_ERR_ARG, "sweep: LDS budget too small for the y/z line store");
     }
-    const long long *pre = g->d_prefix + (size_t)(axis + 1) * (ndom + 1);
-    const long long ntiles = g->prefix[axis + 1][ndom];
+    const int phase = (rest ? kRest0 + 1 : kSweep0) + axis;
+    const long long *pre = g->d_prefix + (size_t)phase * (ndom + 1);
+    const long long ntiles = g->prefix[phase][ndom];
     if (ntiles == 0)
         return BFVMB_OK;
     // default grid: one block per tile, except for the FP32 x variants with register chunks
@@ -1313,18 +1320,18 @@ hipError_t yz_attributes(int bytes)
 
 }  // namespace
 
-int launch_sweep(Group *g, int axis)
+int launch_sweep(Group *g, int axis, bool rest)
 {
     if (g->precision == BFVMB_FP64)
-        return launch_sweep_t<double>(g, axis, false);
-    return launch_sweep_t<float>(g, axis, false);
+        return launch_sweep_t<double>(g, axis, false, rest);
+    return launch_sweep_t<float>(g, axis, false, rest);
 }
 
-int launch_sweep_x_agents(Group *g)
+int launch_sweep_x_agents(Group *g, bool rest)
 {
     if (g->precision != BFVMB_FP64)
         return set_error(g, BFVMB_ERR_STATE, "the fused agent update is an FP64 kernel");
-    return launch_sweep_t<double>(g, 0, true);
+    return launch_sweep_t<double>(g, 0, true, rest);
 }
 
 int sweep_lds_attributes(size_t lds_bytes)

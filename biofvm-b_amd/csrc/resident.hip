@@ -1,0 +1,858 @@
+// resident.hip -- the x and y sweeps of whole z planes held in LDS.
+//
+// The kernels of lod.hip stream a line through a ring of rows and keep of it what fits on chip;
+// they are made for lines and fields far larger than a CU's storage.  Where a z plane of one
+// substrate fits into a CU's LDS (FP64 up to about 139 x 139, FP32 200 x 200), k_plane applies the
+// cell sources and sinks, the x sweep and the y sweep to it there: both sweeps stay inside the
+// plane, so the field crosses the memory system once instead of twice, the agents' voxels are
+// updated without a pass of their own, and a step is two launches (planes, z sweep).
+//
+// What bounds it is the recurrence, one line per lane: at most ceil(lines / 64) wavefronts of a
+// workgroup are at work, and a single wavefront issues about one operation per 6 clocks, dependent
+// or not (LDS latency: 90 clocks).  So what counts is operations per row: a forward row divides by
+// a reciprocal pair (2 operations, div_corr takes 5), a backward row is one operation, and the
+// Thomas tables of a line are staged in LDS beside it and read by broadcast.  (Read by scalar
+// loads, as in lod.hip, they arrived one memory latency per batch late, since a launch starts
+// with cold scalar caches and the compiler sinks such loads to their use: 94 and 90 clocks per
+// forward and backward row of a 128 x 128 FP64 plane instead of 67 and 43.)
+//
+// Microseconds per step of sweeps (separate sweeps -> planes and z sweep; in brackets x + y ->
+// planes): FP64 50^3 x 1 34 -> 20, 97 x 61 x 83 x 3 66 -> 33, 128^3 x 2 78 -> 46 (52 -> 27),
+// 128^3 x 8 194 -> 137 (139 -> 84, 3.2 TB/s of the 5.0 a copy reaches), 139^3 x 8 318 -> 202; FP32
+// 64^3 x 4 34 -> 22, 160^3 x 4 127 -> 105, 200^3 x 2 151 -> 105, 200^3 x 8 448 -> 313.  Every shape
+// tried whose planes fit (16^3 to 200^3, 16 x 16 x 512) was at least as fast.
+//
+// Tried and dropped: whole z lines in LDS, 64 or 32 per workgroup (slower than the z sweep of
+// lod.hip at every size: 128^3 x 2 FP64 step 55 against 49 us); the next plane's loads issued by
+// the solving threads (24 us per 128 x 128 FP64 plane, with loading wavefronts 21); one element
+// per load (k_plane's loaders then overflow the instruction cache in FP32, 190 x 190 planes twice
+// as slow).
+#include <algorithm>
+#include <type_traits>
+
+#include "bfvmb_internal.hpp"
+
+namespace bfvmb {
+namespace {
+
+typedef const __attribute__((address_space(4))) double *ctab;
+__device__ __forceinline__ ctab as_ctab(const double *p) { return (ctab)p; }
+
+// Field values go through the global address space: a generic (flat) access also counts on the
+// LDS counter, so every wait for LDS would drain the next plane's loads.
+template <class T>
+using gmem = __attribute__((address_space(1))) T *;
+template <class T>
+__device__ __forceinline__ gmem<T> as_global(T *p)
+{
+    return (gmem<T>)p;
+}
+
+__device__ __forceinline__ int find_domain(const long long *prefix, int ndom, long long t)
+{
+    int lo = 0, hi = ndom - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (prefix[mid] <= t)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return lo;
+}
+
+// Workgroup barrier that orders LDS only: __syncthreads() also waits for every global access in
+// flight, and with it for the next plane's loads.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// How a forward row divides by its denominator (FP64 storage; FP32 storage multiplies by rden).
+// All three give the correctly rounded quotient for the numerators they are used on.
+enum Division {
+    kPair,  // fma(a, rden, a*rlow): rows with a reciprocal pair (reciprocal_pair, thomas.cpp)
+    kCorr,  // a*rden and two corrections (Markstein): a substrate with a row that has no pair
+    kTrue   // IEEE division: tiny, infinite or NaN numerators
+};
+
+// Key of a numerator that kPair and kCorr must not divide: with h = the upper 32 bits of its
+// pattern, (h << 1) - (kTinyHi << 1) (mod 2^32; the shift drops the sign) is below kKeyBad
+// exactly when 2^-900 <= |a| < inf (below, the low product or the correction's residual may
+// underflow).  A line keeps the largest key it met.
+constexpr unsigned kTinyHi = (1023u - 900u) << 20;
+constexpr unsigned kKeyBad = (0x7ff00000u << 1) - (kTinyHi << 1);
+__device__ __forceinline__ unsigned num_key(double a)
+{
+    unsigned k;  // one operation; from C++ the compiler makes three of it (align, mask, add)
+    asm("v_lshl_add_u32 %0, %1, 1, %2" : "=v"(k) : "v"(__double2hiint(a)), "s"(0u - (kTinyHi << 1)));
+    return k;
+}
+
+// a / den; d1 = rlow (kPair) or den (kCorr, kTrue)
+template <class T, int DIV>
+__device__ __forceinline__ double divide(double a, double d1, double rden)
+{
+    if constexpr (sizeof(T) == 4)
+        return a * rden;
+    else if constexpr (DIV == kPair)
+        return fma(a, rden, a * d1);
+    else if constexpr (DIV == kCorr) {
+        double q = a * rden;
+        q = fma(fma(-q, d1, a), rden, q);
+        return fma(fma(-q, d1, a), rden, q);
+    } else
+        return a / d1;
+}
+
+// Tables of one axis and substrate, staged in LDS: what a forward row divides by ({rlow or den,
+// rden}; FP32 storage: rden) and the back-substitution factor.
+template <class T>
+using FwdRow = std::conditional_t<sizeof(T) == 8, double2, double>;
+template <class T>
+__host__ __device__ constexpr size_t table_bytes()  // per row
+{
+    return sizeof(FwdRow<T>) + sizeof(double);
+}
+template <class T>
+__device__ __forceinline__ void load_row(const AxisTables &tab, size_t off, int n, bool pair, int i, FwdRow<T> &f,
+                                         double &c)
+{
+    const int k = (int)min(i, n - 1);
+    if constexpr (sizeof(T) == 8)
+        f = make_double2(as_global((pair ? tab.rlow : tab.den) + off)[k], as_global(tab.rden + off)[k]);
+    else
+        f = as_global(tab.rden + off)[k];
+    c = as_global(tab.cc + off)[k];
+}
+
+// Rows are taken in batches of kBatch from two buffers, each refilled as soon as its batch is
+// computed, so a batch's rows and table entries are requested one batch of arithmetic before
+// their use, and no more LDS accesses are in flight than the wait counter tells apart (15).
+// Requests past the last batch repeat it.
+template <class T, int kBatch>
+struct Rows {
+    T *q[kBatch];  // where they are
+    T v[kBatch];
+    FwdRow<T> f[kBatch];
+};
+
+// LDS offsets of a line's rows: the columns of a plane (y lines) lie pitch elements apart, plus, in a
+// SKEWed plane, one element every 2^shift rows; x lines are contiguous.  The extra element never
+// falls inside a batch (batches start at multiples of 4, shift >= 2).
+template <bool SKEW>
+struct Columns {
+    int pitch, shift;
+    __host__ __device__ int operator()(int k) const { return SKEW ? k * pitch + (k >> shift) : k * pitch; }
+    __device__ int step() const { return pitch; }
+};
+struct Contiguous {
+    __device__ int operator()(int k) const { return k; }
+    __device__ constexpr int step() const { return 1; }
+};
+
+// One Thomas line in LDS, row k at p[at(k)], swept forward in place.  Returns the last row's value
+// in double; `key` collects num_key (FP64, not kTrue).  The first row of a line may be +0 (a
+// Dirichlet value of 0): every division gives +0 for it, so its numerator is not flagged.
+template <class T, int DIV, int kBatch, class At>
+__device__ __forceinline__ double forward_line(T *p, At at, int n, double c1, const FwdRow<T> *f, ctab den,
+                                               unsigned &key)
+{
+    if constexpr (sizeof(T) == 8 && DIV == kTrue) {  // rare: row by row, few registers
+        double y = -0.0;
+#pragma unroll 1
+        for (int k = 0; k < n; ++k) {
+            y = fma(c1, y, (double)p[at(k)]) / den[k];
+            p[at(k)] = (T)y;
+        }
+        return y;
+    }
+    auto request = [&](int k, Rows<T, kBatch> &r) {
+        r.q[0] = p + at(k);
+#pragma unroll
+        for (int j = 1; j < kBatch; ++j)
+            r.q[j] = r.q[j - 1] + at.step();
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            r.v[j] = *r.q[j];
+            r.f[j] = f[k + j];
+        }
+        asm volatile("" ::: "memory");  // requested here, not where the values are used
+    };
+    double y = -0.0;  // fma(c1, -0.0, v) is v, signed zeros included
+    unsigned kb = 0u;
+    auto row = [&](T *q, T v, const FwdRow<T> &d) {
+        const double num = fma(c1, y, (double)v);
+        if constexpr (sizeof(T) == 8) {
+            kb = max(kb, num_key(num));
+            y = divide<T, DIV>(num, d.x, d.y);
+        } else
+            y = num * d;
+        *q = (T)y;
+    };
+    auto batch = [&](const Rows<T, kBatch> &r) {
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j)
+            row(r.q[j], r.v[j], r.f[j]);
+    };
+    auto few = [&](int k, Rows<T, kBatch> &r) {
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            r.q[j] = p + at(min(k + j, n - 1));
+            r.v[j] = *r.q[j];
+            r.f[j] = f[min(k + j, n - 1)];
+        }
+    };
+    auto some = [&](int k, const Rows<T, kBatch> &r) {  // the rows of a batch that exist
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j)
+            if (k + j < n)
+                row(r.q[j], r.v[j], r.f[j]);
+    };
+    // the first row, then pairs of batches, then the rest
+    Rows<T, kBatch> r0, r1;
+    few(0, r0);
+    const int pairs = n > kBatch ? (n - kBatch) / (2 * kBatch) : 0;
+    const int end = kBatch + pairs * 2 * kBatch;  // first row after the pairs
+    if (pairs > 0)
+        request(kBatch, r1);
+    row(r0.q[0], r0.v[0], r0.f[0]);
+    if constexpr (sizeof(T) == 8)
+        kb = __double_as_longlong((double)r0.v[0]) == 0 ? 0u : kb;
+#pragma unroll
+    for (int j = 1; j < kBatch; ++j)
+        if (j < n)
+            row(r0.q[j], r0.v[j], r0.f[j]);
+    if (pairs > 0) {
+        request(2 * kBatch, r0);
+        for (int k = kBatch; k < end; k += 2 * kBatch) {
+            batch(r1);
+            request(min(k + 2 * kBatch, end - kBatch), r1);
+            batch(r0);
+            request(min(k + 3 * kBatch, end - kBatch), r0);
+        }
+    }
+    if (end < n) {
+        few(end, r0);
+        few(end + kBatch, r1);
+        some(end, r0);
+        some(end + kBatch, r1);
+    }
+    if constexpr (sizeof(T) == 8)
+        key = max(key, kb);
+    return y;
+}
+
+// Back substitution of the same line from its last row's value xv: rows n-2 .. 0 go to out(k, x),
+// in that order (k is wave-uniform).
+template <class T, int kBatch, class At, class Out>
+__device__ __forceinline__ void back_line(const T *p, At at, int n, double xv, const double *c, Out out)
+{
+    struct {
+        T v[kBatch];
+        double c[kBatch];
+    } r0, r1;
+    auto request = [&](int k, auto &r) {  // rows k .. k + kBatch - 1
+        const T *q = p + at(k);
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            r.v[j] = *q;
+            r.c[j] = c[k + j];
+            q += at.step();
+        }
+        asm volatile("" ::: "memory");
+    };
+    auto batch = [&](int k, auto &r) {
+#pragma unroll
+        for (int j = kBatch - 1; j >= 0; --j) {
+            xv = fma(-r.c[j], xv, (double)r.v[j]);
+            out(k + j, xv);
+        }
+    };
+    // rows [0, full) in pairs of batches, [full, n - 1) first
+    const int full = (n - 1) / (2 * kBatch) * (2 * kBatch);
+    auto few = [&](int k, auto &r) {
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            r.v[j] = p[at(min(k + j, n - 1))];
+            r.c[j] = c[min(k + j, n - 1)];
+        }
+    };
+    few(full + kBatch, r1);
+    few(full, r0);
+#pragma unroll
+    for (int j = kBatch - 2; j >= 0; --j)
+        if (full + kBatch + j < n - 1) {
+            xv = fma(-r1.c[j], xv, (double)r1.v[j]);
+            out(full + kBatch + j, xv);
+        }
+    if (full > 0)
+        request(full - kBatch, r1);
+#pragma unroll
+    for (int j = kBatch - 1; j >= 0; --j)
+        if (full + j < n - 1) {
+            xv = fma(-r0.c[j], xv, (double)r0.v[j]);
+            out(full + j, xv);
+        }
+    if (full > 0)
+        request(full - 2 * kBatch, r0);
+    for (int k = full - 2 * kBatch; k >= 0; k -= 2 * kBatch) {
+        batch(k + kBatch, r1);
+        request(max(k - kBatch, 0), r1);
+        batch(k, r0);
+        request(max(k - 2 * kBatch, 0), r0);
+    }
+}
+
+// results are stored plainly: the z sweep reads them next, often from the 256 MB memory-side cache
+template <class T>
+__device__ __forceinline__ void store_result(gmem<T> p, T v)
+{
+    *p = v;
+}
+
+// n / d with inv = ceil(2^32 / d), d >= 2: exact while n*d < 2^32 (planes in LDS hold at most 2^15.4
+// values)
+__device__ __forceinline__ int quot(int n, unsigned inv) { return (int)__umulhi((unsigned)n, inv); }
+__device__ __forceinline__ unsigned quot_inv(int d) { return 0xffffffffu / (unsigned)d + 1u; }
+
+// Layout of a plane in LDS: row y at y*pitch, or (SKEW) y*nx + (y >> shift).  64 rows read at one
+// column (x sweep) have to fall on distinct banks, 32 of 4 bytes for each group of lanes served at
+// once (32 lanes of 4 bytes, 16 of 8): an odd pitch does that.  Where rows of nx + 1 do not fit, one
+// element more every group/g rows does too, g = gcd(nx, group) the number of rows apart by a
+// multiple of all banks; a 200 x 200 FP32 plane fits that way.  It is not the rule because the
+// column sweep then forms longer addresses (128 x 128 FP64 planes: 4% slower).
+template <bool SKEW>
+__host__ __device__ __forceinline__ Columns<SKEW> plane_layout(int nx, size_t elem)
+{
+    if (!SKEW)
+        return Columns<SKEW>{nx | 1, 0};
+    const int group = elem == 8 ? 16 : 32;
+    int g = 1, shift = elem == 8 ? 4 : 5;
+    while (g < group && nx % (2 * g) == 0) {
+        g *= 2;
+        --shift;
+    }
+    return Columns<SKEW>{nx, shift};
+}
+
+constexpr int kVoteBytes = 16;  // before the tile in LDS
+
+constexpr int kMaxThreads = 512;
+
+// The kernel comes in two sizes.  BIG, planes above 80 KB: one workgroup per CU, 256 registers per
+// lane.  Otherwise 128 (FP64) or 96 registers, so that several workgroups share a CU, with smaller
+// batches of rows.  Pairs of a plane's elements per loading thread, all of them in registers at
+// once (pairs, aligned like one element, so that the unrolled loads fit the instruction cache: a
+// 76 KB kernel of single FP32 loads ran at half the speed):
+template <class T, bool BIG>
+constexpr int plane_loads()
+{
+    return (BIG ? (sizeof(T) == 8 ? 31 : 80) : (sizeof(T) == 8 ? 15 : 24));
+}
+template <class T>
+struct PairOf;
+template <>
+struct PairOf<double> {
+    typedef double type __attribute__((ext_vector_type(2), aligned(8)));
+};
+template <>
+struct PairOf<float> {
+    typedef float type __attribute__((ext_vector_type(2), aligned(4)));
+};
+template <class T, bool BIG>
+constexpr int plane_waves_per_simd()
+{
+    return BIG ? 2 : sizeof(T) == 8 ? 4 : 5;
+}
+
+// What a workgroup needs to know of one plane.
+template <class T>
+struct Plane {
+    const DomainDesc<T> *D;
+    int di, s, z;
+};
+
+template <class T>
+__device__ __forceinline__ Plane<T> locate(const DomainDesc<T> *descs, const long long *prefix, int ndom, int t)
+{
+    Plane<T> p;
+    long long lt = t;
+    p.di = 0;
+    if (ndom > 1) {
+        p.di = __builtin_amdgcn_readfirstlane(find_domain(prefix, ndom, lt));
+        lt -= prefix[p.di];
+    }
+    p.D = descs + p.di;
+    const int nz = p.D->nz;
+    p.s = __builtin_amdgcn_readfirstlane((int)((unsigned)lt / (unsigned)nz));
+    p.z = __builtin_amdgcn_readfirstlane((int)lt - p.s * nz);
+    return p;
+}
+
+// Workgroups stride over the z planes of a size class; a plane of one substrate is held in LDS,
+// (rows as plane_layout places them), and swept in place there: x then y, or y then x for the adjoint's
+// reverse order (YX).  AG: the cell sources and sinks first, on the plane in LDS (segments
+// [zseg[z], zseg[z+1]) of the voxel-sorted agent list), agents of a voxel in list order, as the
+// separate agent kernel applies them.  The plane is written back where it was read.
+//
+// The first `solvers` threads (whole wavefronts, at least as many lanes as the plane has rows or
+// columns) sweep; the other wavefronts load: they read the next plane into registers while this
+// one is swept, and put it into LDS when it is done.  (Registers, because LDS is full; wavefronts
+// of their own, because the solvers' registers and instruction slots are what a plane waits
+// for.)  Both run through the same sequence of barriers.
+template <class T, bool BIG, bool SKEW, bool YX, bool AG>
+__global__ __launch_bounds__(kMaxThreads, (plane_waves_per_simd<T, BIG>())) void k_plane(const DomainDesc<T> *__restrict__ descs,
+                                                                    const long long *__restrict__ prefix, int ndom,
+                                                                    int planes, int solvers, int parity)
+{
+    constexpr int kLoads = plane_loads<T, BIG>(), B = BIG || sizeof(T) == 4 ? 4 : 2;
+    extern __shared__ unsigned char smem[];
+    int *vote = reinterpret_cast<int *>(smem);  // set by a lane that met a flagged numerator
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int wave_first = __builtin_amdgcn_readfirstlane(tid);  // uniform: this wavefront's role
+
+    // LDS: vote, tables of the axis being swept, plane
+    auto lds_tables = [&](const DomainDesc<T> &) { return reinterpret_cast<FwdRow<T> *>(smem + kVoteBytes); };
+    auto lds_factors = [&](const DomainDesc<T> &D) {
+        return reinterpret_cast<double *>(lds_tables(D) + max(D.nx, D.ny));
+    };
+    auto lds_plane = [&](const DomainDesc<T> &D) { return reinterpret_cast<T *>(lds_factors(D) + max(D.nx, D.ny)); };
+    // LDS index of the plane's element e
+    auto at = [](int e, int nx, const Columns<SKEW> &lay, unsigned inv) {
+        if (lay.pitch == nx && !SKEW)
+            return e;
+        const int y = quot(e, inv);
+        return e + (SKEW ? y >> lay.shift : y);
+    };
+    auto active = [&](const DomainDesc<T> &D, int s) {
+        return __builtin_amdgcn_readfirstlane((int)as_global(D.dact)[s]) != 0;
+    };
+    // results that went to LDS, out by all threads
+    auto copy_out = [&](const DomainDesc<T> &D, int s, int z) {
+        const int nel = D.nx * D.ny;
+        const Columns<SKEW> lay = plane_layout<SKEW>(D.nx, sizeof(T));
+        const unsigned inv = quot_inv(max(D.nx, 2));
+        const T *P = lds_plane(D);
+        const gmem<T> f = as_global(D.field[parity] + ((size_t)s * D.nz + z) * nel);
+        for (int e = tid; e < nel; e += nt)
+            store_result<T>(f + e, P[at(e, D.nx, lay, inv)]);
+    };
+
+    if (wave_first >= solvers) {
+        // ------------------------------------------------------------------ loading wavefronts
+        const int lid = tid - solvers, ln = nt - solvers;
+        typedef typename PairOf<T>::type Pair;
+        Pair r[kLoads];  // the next plane's values
+        // first element of pair lid + j*ln, the last pair's for lanes past the end (n >= 2)
+        auto first = [&](int j, int n) { return min(2 * (lid + j * ln), n - 2); };
+        auto request = [&](const Plane<T> &p) {
+            const int n = p.D->nx * p.D->ny;
+            const gmem<const T> src = as_global<const T>(p.D->field[parity] + ((size_t)p.s * p.D->nz + p.z) * n);
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+                if (2 * j * ln < n)
+                    r[j] = *(gmem<const Pair>)(src + (unsigned)first(j, n));
+        };
+        int t = blockIdx.x;
+        Plane<T> p = locate(descs, prefix, ndom, t);
+        request(p);
+        for (;;) {
+            const DomainDesc<T> &D = *p.D;
+            const int s = p.s, z = p.z, nel = D.nx * D.ny;
+            const bool act = active(D, s), voxels = D.dface != nullptr;
+            const bool zface = act && (z == 0 || z == D.nz - 1);
+            {
+                T *P = lds_plane(D);
+                const Columns<SKEW> lay = plane_layout<SKEW>(D.nx, sizeof(T));
+                const unsigned inv = quot_inv(max(D.nx, 2));
+#pragma unroll
+                for (int j = 0; j < kLoads; ++j)
+                    if (2 * j * ln < nel) {
+                        int e = first(j, nel);
+                        asm("" : "+v"(e));  // so many LDS addresses are cheaper to form than to keep
+                        // the pair stays together: rows are padded where nx is even, and then a
+                        // pair does not cross a row's end
+                        T *q = P + at(e, D.nx, lay, inv);
+                        q[0] = r[j].x;
+                        q[1] = r[j].y;
+                    }
+            }
+            lds_barrier();  // plane and first tables in LDS
+            t += gridDim.x;
+            if (t < planes) {
+                p = locate(descs, prefix, ndom, t);
+                request(p);
+            }
+            if (!zface) {
+                if (AG && D.zseg != nullptr)
+                    lds_barrier();  // agents
+                for (bool exact = false;;) {
+                    if (act)
+                        lds_barrier();  // Dirichlet values
+                    lds_barrier();      // first axis
+                    lds_barrier();      // Dirichlet values, second tables
+                    if constexpr (sizeof(T) == 8) {
+                        if (!exact) {
+                            lds_barrier();  // vote
+                            if (*vote) {
+                                exact = true;
+                                lds_barrier();  // vote read
+                                lds_barrier();  // plane reloaded
+                                if (AG && D.zseg != nullptr)
+                                    lds_barrier();
+                                continue;
+                            }
+                        }
+                    }
+                    if (YX || (act && voxels)) {
+                        lds_barrier();  // second axis
+                        if (act)
+                            lds_barrier();
+                        copy_out(D, s, z);
+                    }
+                    break;
+                }
+            }
+            if (t >= planes)
+                return;
+            lds_barrier();  // the plane's LDS is free
+        }
+    }
+
+    // ---------------------------------------------------------------------- solving wavefronts
+    FwdRow<T> xf, yf;  // row tid of the tables
+    double xc = 0.0, yc = 0.0;
+    if (tid == 0)
+        *vote = 0;
+    int t = blockIdx.x, di_had = -1, s_had = -1;
+    for (;;) {
+        const Plane<T> p = locate(descs, prefix, ndom, t);
+        const DomainDesc<T> &D = *p.D;
+        const int s = p.s, z = p.z;
+        const int nx = D.nx, ny = D.ny, nz = D.nz;
+        const int nel = nx * ny;
+        const Columns<SKEW> lay = plane_layout<SKEW>(nx, sizeof(T));
+        const unsigned inv = quot_inv(max(nx, 2));
+        const double c1 = as_ctab(D.c1)[s];
+        const bool pairx = sizeof(T) == 4 || as_ctab(D.tab[0].nopair)[s] == 0.0;
+        const bool pairy = sizeof(T) == 4 || as_ctab(D.tab[1].nopair)[s] == 0.0;
+        const bool act = active(D, s);
+        const T dv = ((const __attribute__((address_space(4))) T *)D.dval)[s];
+        const gmem<const T> fv = as_global(D.dface);  // per-voxel Dirichlet values
+        const bool voxels = D.dface != nullptr;
+        const gmem<T> f = as_global(D.field[parity] + ((size_t)s * nz + z) * nel);
+        if (p.di != di_had || s != s_had) {
+            load_row<T>(D.tab[0], (size_t)s * nx, nx, pairx, tid, xf, xc);
+            load_row<T>(D.tab[1], (size_t)s * ny, ny, pairy, tid, yf, yc);
+            di_had = p.di;
+            s_had = s;
+        }
+        FwdRow<T> *tf = lds_tables(D);
+        double *tc = lds_factors(D);
+        T *P = lds_plane(D);
+        auto put_table = [&](bool x) {
+            if (tid < (x ? nx : ny)) {
+                tf[tid] = x ? xf : yf;
+                tc[tid] = x ? xc : yc;
+            }
+        };
+        // the plane's face voxels take their Dirichlet values (apply_dirichlet_conditions)
+        auto dirichlet = [&]() {
+            if (!act)
+                return;
+            // low or high face of y (k < nx) or x, position k along it
+            auto place = [&](int e, int k) {
+                return P + (k < nx ? lay(e ? ny - 1 : 0) + k : lay(k - nx) + (e ? nx - 1 : 0));
+            };
+            if (voxels)
+                for (int i = tid; i < 2 * (nx + ny); i += solvers) {
+                    const int e = i & 1, k = i >> 1;
+                    *place(e, k) = fv[k < nx ? face_y(nx, ny, nz, D.nsub, e, s, k, z)
+                                             : face_x(ny, nz, D.nsub, e, s, k - nx, z)];
+                }
+            else
+                for (int i = tid; i < 2 * (nx + ny); i += solvers)
+                    *place(i & 1, i >> 1) = dv;
+        };
+        auto agents = [&]() {
+            const auto zs = (const __attribute__((address_space(4))) int *)D.zseg;
+            const int lo = zs[z], hi = zs[z + 1];
+            const gmem<const double> a1 = as_global(D.t1 + (size_t)s * D.nact), a2 = as_global(D.t2 + (size_t)s * D.nact);
+            for (int k = lo + tid; k < hi; k += solvers) {
+                const int e = at((int)(as_global(D.seg_off)[k] - (long long)z * nel), nx, lay, inv);
+                const int b1 = as_global(D.seg_start)[k + 1];
+                double v = (double)P[e];
+                for (int a = as_global(D.seg_start)[k]; a < b1; ++a) {
+                    v = v + a1[a];
+                    v = v / a2[a];
+                }
+                P[e] = (T)v;
+            }
+        };
+        const bool zface = act && (z == 0 || z == nz - 1);  // such a plane ends as its Dirichlet values
+        put_table(!YX);
+        lds_barrier();  // plane and first tables in LDS
+        if (zface) {
+            const size_t fz = face_z(nx, ny, nz, D.nsub, z == 0 ? 0 : 1, s, 0, 0);
+            if (voxels)
+                for (int e = tid; e < nel; e += solvers)
+                    f[e] = fv[fz + e];
+            else
+                for (int e = tid; e < nel; e += solvers)
+                    f[e] = dv;
+        } else {
+            if (AG && D.zseg != nullptr) {
+                agents();
+                lds_barrier();
+            }
+            for (bool exact = false;;) {
+                if (act) {
+                    dirichlet();
+                    lds_barrier();
+                }
+                unsigned key = 0u;
+                auto forward = [&](T *q, auto rows, int n, bool pair, const double *den) {
+                    if constexpr (sizeof(T) == 4)
+                        return forward_line<T, kPair, B>(q, rows, n, c1, tf, nullptr, key);
+                    else
+                        return exact ? forward_line<T, kTrue, B>(q, rows, n, c1, tf, as_ctab(den), key)
+                                     : pair ? forward_line<T, kPair, B>(q, rows, n, c1, tf, nullptr, key)
+                                            : forward_line<T, kCorr, B>(q, rows, n, c1, tf, nullptr, key);
+                };
+                const Contiguous row;
+                // a line on a Dirichlet face is overwritten whole, whatever its numerators were
+                auto x_forward = [&]() {
+                    const unsigned k0 = key;
+                    const double y = forward(P + lay(tid), row, nx, pairx, D.tab[0].den + (size_t)s * nx);
+                    if (act && (tid == 0 || tid == ny - 1))
+                        key = k0;
+                    return y;
+                };
+                auto x_back = [&](double y) {
+                    T *q = P + lay(tid);
+                    back_line<T, B>(q, row, nx, y, tc, [&](int k, double x) { q[k] = (T)x; });
+                };
+                auto y_forward = [&]() {
+                    const unsigned k0 = key;
+                    const double y = forward(P + tid, lay, ny, pairy, D.tab[1].den + (size_t)s * ny);
+                    if (act && (tid == 0 || tid == nx - 1))
+                        key = k0;
+                    return y;
+                };
+                auto y_back = [&](double y) {
+                    T *q = P + tid;
+                    back_line<T, B>(q, lay, ny, y, tc, [&](int k, double x) { q[lay(k)] = (T)x; });
+                };
+                double last = 0.0;
+                if constexpr (!YX) {
+                    if (tid < ny)
+                        x_back(x_forward());
+                } else {
+                    if (tid < nx)
+                        y_back(y_forward());
+                }
+                lds_barrier();  // first axis
+                dirichlet();
+                put_table(YX);
+                lds_barrier();
+                if constexpr (!YX) {
+                    if (tid < nx)
+                        last = y_forward();
+                } else {
+                    if (tid < ny)
+                        last = x_forward();
+                }
+                if constexpr (sizeof(T) == 8) {
+                    // a numerator outside the fast divisions' range somewhere in the plane: the
+                    // whole plane again from memory (nothing is stored yet) with true divisions
+                    if (!exact) {
+                        if (key >= kKeyBad)
+                            *vote = 1;
+                        lds_barrier();
+                        if (*vote) {
+                            exact = true;
+                            lds_barrier();
+                            if (tid == 0)
+                                *vote = 0;
+                            for (int e = tid; e < nel; e += solvers)
+                                P[at(e, nx, lay, inv)] = f[e];
+                            put_table(!YX);
+                            lds_barrier();
+                            if (AG && D.zseg != nullptr) {
+                                agents();
+                                lds_barrier();
+                            }
+                            continue;
+                        }
+                    }
+                }
+                if (!YX && !(act && voxels)) {  // results go out as they are found, one row of columns at a time
+                    if (tid < nx) {
+                        const bool face = act && (tid == 0 || tid == nx - 1);
+                        gmem<T> q = f + tid + (size_t)(ny - 1) * nx;  // rows are stored from the last to the first
+                        store_result<T>(q, act ? dv : (T)last);
+                        back_line<T, B>(P + tid, lay, ny, last, tc, [&](int k, double x) {
+                            q -= nx;
+                            store_result<T>(q, face || (act && k == 0) ? dv : (T)x);
+                        });
+                    }
+                    break;
+                }
+                if constexpr (YX) {
+                    if (tid < ny)
+                        x_back(last);
+                } else {
+                    if (tid < nx)
+                        y_back(last);
+                }
+                lds_barrier();  // second axis
+                if (act) {
+                    dirichlet();
+                    lds_barrier();
+                }
+                copy_out(D, s, z);
+                break;
+            }
+        }
+        t += gridDim.x;
+        if (t >= planes)
+            return;
+        lds_barrier();  // the plane's LDS is free
+    }
+}
+
+template <bool SKEW>
+size_t plane_bytes(const Domain &d, size_t elem)
+{
+    const size_t row = elem == 8 ? table_bytes<double>() : table_bytes<float>();
+    return kVoteBytes + (size_t)std::max(d.nx, d.ny) * row + (size_t)(plane_layout<SKEW>(d.nx, elem)(d.ny) + 1) * elem;
+}
+
+int size_class(size_t bytes)
+{
+    int c = 0;
+    while (c < 3 && bytes > (kLdsBytes >> (3 - c)))
+        ++c;
+    return c;
+}
+
+// loading threads for planes of `el` elements, at most `loads` pairs each (whole wavefronts)
+size_t plane_loaders(size_t el, int loads) { return ((el + 2 * loads - 1) / (2 * loads) + kWave - 1) / kWave * kWave; }
+
+constexpr int kSmallClasses = 3;  // classes of the small kernel: planes up to 80 KB
+constexpr int kSkewClass = 4;     // planes that fit only skewed
+static_assert(kClasses == kSkewClass + 1, "size classes");
+
+template <class T, bool BIG, bool SKEW, bool YX, bool AG>
+void launch_plane_kernel(const Group *g, int c, unsigned grid, int planes, unsigned threads, int solvers, size_t lds)
+{
+    const DomainDesc<T> *d = static_cast<const DomainDesc<T> *>(g->d_desc);
+    const int ndom = (int)g->doms.size();
+    const long long *pre = g->d_prefix + (size_t)(kPlane0 + c) * (ndom + 1);
+    hipLaunchKernelGGL((k_plane<T, BIG, SKEW, YX, AG>), dim3(grid), dim3(threads), lds, g->stream, d, pre, ndom, planes,
+                       solvers, g->cur);
+}
+
+template <class T, bool BIG, bool SKEW>
+int launch_planes_class(Group *g, int c, bool yx, bool agents)
+{
+    const long long planes = g->prefix[kPlane0 + c][g->doms.size()];
+    size_t lds = 0, el = 0;
+    int lines = 0;
+    for (const Domain &d : g->doms)
+        if (d.plane_class == c) {
+            lds = std::max(lds, plane_bytes<SKEW>(d, sizeof(T)));
+            el = std::max(el, (size_t)d.nx * d.ny);
+            lines = std::max(lines, std::max(d.nx, d.ny));
+        }
+    const int solvers = (lines + kWave - 1) / kWave * kWave;
+    const unsigned th = BIG ? kMaxThreads : (unsigned)(solvers + plane_loaders(el, plane_loads<T, BIG>()));
+    // as many workgroups as the CUs hold, each striding over the planes
+    const int waves = 4 * plane_waves_per_simd<T, BIG>() / (int)(th / kWave);
+    const long long percu = std::max(1, std::min(waves, (int)(kLdsBytes / lds)));
+    const unsigned grid = (unsigned)std::min<long long>(planes, percu * std::max(g->cu_count, 1));
+    if (yx)
+        launch_plane_kernel<T, BIG, SKEW, true, false>(g, c, grid, (int)planes, th, solvers, lds);
+    else if (agents)
+        launch_plane_kernel<T, BIG, SKEW, false, true>(g, c, grid, (int)planes, th, solvers, lds);
+    else
+        launch_plane_kernel<T, BIG, SKEW, false, false>(g, c, grid, (int)planes, th, solvers, lds);
+    return hip_check(g, hipGetLastError(), "plane launch");
+}
+
+template <class T>
+int launch_planes_t(Group *g, bool yx, bool agents)
+{
+    for (int c = 0; c < kClasses; ++c) {
+        if (g->prefix[kPlane0 + c].back() == 0)
+            continue;
+        const int rc = c < kSmallClasses ? launch_planes_class<T, false, false>(g, c, yx, agents)
+                       : c < kSkewClass  ? launch_planes_class<T, true, false>(g, c, yx, agents)
+                                         : launch_planes_class<T, true, true>(g, c, yx, agents);
+        if (rc)
+            return rc;
+    }
+    return BFVMB_OK;
+}
+
+template <class T, bool BIG, bool SKEW>
+hipError_t attributes(int bytes)
+{
+    const void *k[3] = {(const void *)k_plane<T, BIG, SKEW, false, false>, (const void *)k_plane<T, BIG, SKEW, false, true>,
+                        (const void *)k_plane<T, BIG, SKEW, true, false>};
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < 3 && e == hipSuccess; ++i)
+        e = hipFuncSetAttribute(k[i], hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    return e;
+}
+
+template <class T>
+hipError_t attributes_all(int bytes)
+{
+    hipError_t e = attributes<T, false, false>(bytes);
+    if (e == hipSuccess)
+        e = attributes<T, true, false>(bytes);
+    if (e == hipSuccess)
+        e = attributes<T, true, true>(bytes);
+    return e;
+}
+
+}  // namespace
+
+void resident_class(const Group *g, Domain &d)
+{
+    const size_t limit = std::min(kLdsBytes, g->max_lds_per_block), el = (size_t)d.nx * d.ny;
+    const size_t plain = plane_bytes<false>(d, g->elem), skewed = plane_bytes<true>(d, g->elem);
+    const bool skewable = plane_layout<true>(d.nx, g->elem).shift >= 2;
+    int c = plain <= limit ? size_class(plain) : skewed <= limit && skewable ? kSkewClass : -1;
+    if (c >= 0) {
+        const int loads = g->elem == 8 ? (c < kSmallClasses ? plane_loads<double, false>() : plane_loads<double, true>())
+                                       : (c < kSmallClasses ? plane_loads<float, false>() : plane_loads<float, true>());
+        const size_t solvers = (std::max(d.nx, d.ny) + kWave - 1) / kWave * kWave;
+        if (el < 2 || solvers + plane_loaders(el, loads) > kMaxThreads || (long long)d.nz * d.nsub >= (1LL << 30))
+            c = -1;
+    }
+    d.plane_class = c;
+}
+
+int launch_planes(Group *g, bool yx, bool agents)
+{
+    int rc = sync_descriptors(g);
+    if (rc)
+        return rc;
+    return g->precision == BFVMB_FP64 ? launch_planes_t<double>(g, yx, agents) : launch_planes_t<float>(g, yx, agents);
+}
+
+int resident_lds_attributes(size_t lds_bytes)
+{
+    const int bytes = (int)std::min(lds_bytes, kLdsBytes);
+    hipError_t e = attributes_all<double>(bytes);
+    if (e == hipSuccess)
+        e = attributes_all<float>(bytes);
+    return (int)e;
+}
+
+}  // namespace bfvmb

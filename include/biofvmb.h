@@ -166,12 +166,13 @@ int bfvmb_simulate_diffusion_decay(bfvmb_ctx *ctx, int nsteps);
 
 /* nsteps of the demo time loop (complete_diffusion_demo.cpp:489-493): per step, cell
  * sources/sinks then one LOD step (preceded by the bulk update when bulk rates are set).
- * In FP64 the sources/sinks run inside the x sweep's launch unless some x-sweep tile (64
+ * Where a z plane of a substrate fits into a CU's LDS (FP64 up to about 139 x 139, FP32
+ * 200 x 200), sources/sinks and the x and y sweeps are one launch over planes.  Elsewhere, in FP64 the sources/sinks run inside the x sweep's launch unless some x-sweep tile (64
  * rows y,z) holds more than 3072 occupied voxels; either way the results are those of the
  * two separate calls, bit for bit. */
 int bfvmb_run(bfvmb_ctx *ctx, int nsteps);
 
-/* bfvmb_run captured once as a HIP graph (nsteps x 4 kernel nodes) and replayed as one
+/* bfvmb_run captured once as a HIP graph (nsteps x 2 to 5 kernel nodes) and replayed as one
  * launch; the graph is cached per (nsteps, buffer parity) until agents, coefficients
  * pointers or launch shapes change.  Same results as bfvmb_run. */
 int bfvmb_run_graph(bfvmb_ctx *ctx, int nsteps);
@@ -180,7 +181,8 @@ int bfvmb_run_graph(bfvmb_ctx *ctx, int nsteps);
 int bfvmb_sync(bfvmb_ctx *ctx);
 
 /* One kernel of the step, for measurement: phase 0 = sources/sinks, 1 = x, 2 = y, 3 = z
- * sweep, 4 = sources/sinks and x sweep as bfvmb_run launches them (FP64 with no x-sweep tile
+ * sweep, 4 = sources/sinks and x sweep as bfvmb_run launches them where it sweeps x and y
+ * separately (FP64 with no x-sweep tile
  * of more than 3072 occupied voxels: one fused launch; otherwise phases 0 and 1); enqueued
  * `count` times on the context's stream. */
 int bfvmb_launch_phase(bfvmb_ctx *ctx, int phase, int count);
@@ -192,14 +194,15 @@ int bfvmb_launch_phase(bfvmb_ctx *ctx, int phase, int count);
  * wavefronts share one CU's LDS line store, and rows in flight per lane (y/z: 16/32/64) or
  * the x-sweep kernel variant (FP32: 1 = one column chunk in flight and 17 register chunks,
  * 3 = three chunks in flight and none, each with its Thomas tables read by scalar loads;
- * 2 and 4 = the same with the tables staged in LDS).  Used by the autotuner; results do
+ * 2 and 4 = the same with the tables staged in LDS).  A shape set for x or y also keeps
+ * bfvmb_run's sweeps separate where planes fit into LDS.  Used by the autotuner; results do
  * not depend on it. */
 int bfvmb_set_launch(bfvmb_ctx *ctx, int sweep, int grid_blocks, int lds_blocks_per_cu, int ring_depth);
 
 /* Autotuner: times the candidate launch shapes of each sweep (LDS wavefronts per CU 2, 3,
  * 4, 6, 8; ring depth 32/64 for y/z; the FP32 x variants; one block per tile or a grid of
  * one block per wavefront slot striding over the tiles) over `reps` launches with HIP
- * events and keeps the fastest.
+ * events and keeps the fastest; then x + y at their best shapes against the launch over planes.
  * The field is saved and restored, so tuning does not advance the simulation.  `chosen`
  * (may be NULL) receives 3 x {wavefronts per CU, ring, microseconds per launch}. */
 int bfvmb_autotune(bfvmb_ctx *ctx, int reps, int *chosen);
