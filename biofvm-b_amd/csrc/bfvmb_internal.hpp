@@ -46,6 +46,7 @@ struct AxisTables {
     const double *rden;  // RN(1/den)
     const double *rlow;  // low part of 1/den: fma(a, rden, a*rlow) is RN(a/den) (reciprocal_pair)
     const double *nopair;  // [nsub] number of rows without such a pair
+    const double *settled;  // [nsub] first of the rows, up to n - 2, that all have the same entries
 };
 
 // Device descriptor of one domain (plain data, copied to the GPU).
@@ -105,7 +106,7 @@ struct Domain {
     double dx = 0.0;
     size_t nvox = 0;
     void *field[2] = {nullptr, nullptr};
-    double *coef = nullptr;  // c1[nsub] | per axis den, cc, rden, rlow [nsub][n], nopair [nsub]
+    double *coef = nullptr;  // c1[nsub] | per axis den, cc, rden, rlow [nsub][n], nopair, settled [nsub]
     bool have_coef = false;
     double dt = 0.0;
     std::vector<double> D, decay;
@@ -136,7 +137,7 @@ struct Domain {
 
 // Offsets inside a domain's coefficient block, in doubles.
 struct CoefLayout {
-    size_t c1, den[3], cc[3], rden[3], rlow[3], nopair[3], total;
+    size_t c1, den[3], cc[3], rden[3], rlow[3], nopair[3], settled[3], total;
 };
 CoefLayout coef_layout(const Domain &d);
 

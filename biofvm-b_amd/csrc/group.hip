@@ -43,6 +43,8 @@ CoefLayout coef_layout(const Domain &d)
         off += s * n[a];
         L.nopair[a] = off;
         off += s;
+        L.settled[a] = off;
+        off += s;
     }
     L.total = off + 16;  // scalar loads read a batch of entries at a time
     return L;
@@ -95,7 +97,7 @@ std::vector<DomainDesc<T>> build_descs(Group *g)
             e.c1 = d.coef + L.c1;
             for (int a = 0; a < 3; ++a)
                 e.tab[a] = AxisTables{d.coef + L.den[a], d.coef + L.cc[a], d.coef + L.rden[a], d.coef + L.rlow[a],
-                                      d.coef + L.nopair[a]};
+                                      d.coef + L.nopair[a], d.coef + L.settled[a]};
         }
         e.dval = static_cast<const T *>(d.d_dval);
         e.dact = d.d_dact;
@@ -332,6 +334,13 @@ int domain_set_coefficients(Group *g, int i, const double *D, const double *deca
     for (int a = 0; a < 3; ++a) {
         std::vector<double> den((size_t)ns * n[a]), cc((size_t)ns * n[a]);
         thomas_axis(n[a], ns, c1.data(), c2.data(), c3.data(), c3a.data(), den.data(), cc.data());
+        for (int s = 0; s < ns; ++s) {  // the last row has a coefficient of its own
+            const double *d0 = &den[(size_t)s * n[a]], *c0 = &cc[(size_t)s * n[a]];
+            int k = std::max(n[a] - 2, 0);
+            while (k > 0 && d0[k - 1] == d0[k] && c0[k - 1] == c0[k])
+                --k;
+            blob[L.settled[a] + s] = k;
+        }
         for (size_t k = 0; k < den.size(); ++k) {
             blob[L.den[a] + k] = den[k];
             blob[L.cc[a] + k] = cc[k];

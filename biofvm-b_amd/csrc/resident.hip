@@ -17,16 +17,20 @@
 // forward and backward row of a 128 x 128 FP64 plane instead of 67 and 43.)
 //
 // Microseconds per step of sweeps (separate sweeps -> planes and z sweep; in brackets x + y ->
-// planes): FP64 50^3 x 1 34 -> 20, 97 x 61 x 83 x 3 66 -> 33, 128^3 x 2 78 -> 46 (52 -> 27),
-// 128^3 x 8 194 -> 137 (139 -> 84, 3.2 TB/s of the 5.0 a copy reaches), 139^3 x 8 318 -> 202; FP32
-// 64^3 x 4 34 -> 22, 160^3 x 4 127 -> 105, 200^3 x 2 151 -> 105, 200^3 x 8 448 -> 313.  Every shape
+// planes): FP64 50^3 x 1 34 -> 20, 97 x 61 x 83 x 3 66 -> 32, 128^3 x 2 79 -> 44 (53 -> 25),
+// 128^3 x 8 193 -> 128 (138 -> 77, 3.5 TB/s of the 5.0 a copy reaches), 139^3 x 8 317 -> 195; FP32
+// 64^3 x 4 33 -> 22, 160^3 x 4 127 -> 100, 200^3 x 2 150 -> 100, 200^3 x 8 448 -> 296.  Every shape
 // tried whose planes fit (16^3 to 200^3, 16 x 16 x 512) was at least as fast.
+//
+// The tables of settled rows (forward_line) are kept in registers; read from LDS for every row:
+// 128^3 x 2 FP64 46, 128^3 x 8 137, 200^3 x 8 FP32 313.
 //
 // Tried and dropped: whole z lines in LDS, 64 or 32 per workgroup (slower than the z sweep of
 // lod.hip at every size: 128^3 x 2 FP64 step 55 against 49 us); the next plane's loads issued by
 // the solving threads (24 us per 128 x 128 FP64 plane, with loading wavefronts 21); one element
 // per load (k_plane's loaders then overflow the instruction cache in FP32, 190 x 190 planes twice
-// as slow).
+// as slow); the last sweep's results to LDS and out by all wavefronts instead of a row at a time by
+// the solvers (200^3 x 8 FP32 340 instead of 296).
 #include <algorithm>
 #include <type_traits>
 
@@ -156,8 +160,12 @@ struct Contiguous {
 // One Thomas line in LDS, row k at p[at(k)], swept forward in place.  Returns the last row's value
 // in double; `key` collects num_key (FP64, not kTrue).  The first row of a line may be +0 (a
 // Dirichlet value of 0): every division gives +0 for it, so its numerator is not flagged.
+//
+// The recursion behind the tables settles on one value after some rows (D = 1e3 to 1e5 um^2/min,
+// dt = 0.01, dx = 20: 6 to 30 rows): rows [settled, n - 2] share their entries, which then stay in
+// registers.
 template <class T, int DIV, int kBatch, class At>
-__device__ __forceinline__ double forward_line(T *p, At at, int n, double c1, const FwdRow<T> *f, ctab den,
+__device__ __forceinline__ double forward_line(T *p, At at, int n, int settled, double c1, const FwdRow<T> *f, ctab den,
                                                unsigned &key)
 {
     if constexpr (sizeof(T) == 8 && DIV == kTrue) {  // rare: row by row, few registers
@@ -169,7 +177,7 @@ __device__ __forceinline__ double forward_line(T *p, At at, int n, double c1, co
         }
         return y;
     }
-    auto request = [&](int k, Rows<T, kBatch> &r) {
+    auto request = [&](int k, Rows<T, kBatch> &r, bool table) {
         r.q[0] = p + at(k);
 #pragma unroll
         for (int j = 1; j < kBatch; ++j)
@@ -177,7 +185,8 @@ __device__ __forceinline__ double forward_line(T *p, At at, int n, double c1, co
 #pragma unroll
         for (int j = 0; j < kBatch; ++j) {
             r.v[j] = *r.q[j];
-            r.f[j] = f[k + j];
+            if (table)
+                r.f[j] = f[k + j];
         }
         asm volatile("" ::: "memory");  // requested here, not where the values are used
     };
@@ -211,13 +220,15 @@ __device__ __forceinline__ double forward_line(T *p, At at, int n, double c1, co
             if (k + j < n)
                 row(r.q[j], r.v[j], r.f[j]);
     };
-    // the first row, then pairs of batches, then the rest
+    // the first batch, pairs of batches up to the settled rows, pairs of those, then the rest
     Rows<T, kBatch> r0, r1;
     few(0, r0);
     const int pairs = n > kBatch ? (n - kBatch) / (2 * kBatch) : 0;
-    const int end = kBatch + pairs * 2 * kBatch;  // first row after the pairs
-    if (pairs > 0)
-        request(kBatch, r1);
+    const int early = min(pairs, max(settled - kBatch + 2 * kBatch - 1, 0) / (2 * kBatch));
+    const int same = kBatch + early * 2 * kBatch;  // first settled row taken as one
+    const int late = max(n - 1 - same, 0) / (2 * kBatch), end = same + late * 2 * kBatch;
+    if (early > 0)
+        request(kBatch, r1, true);
     row(r0.q[0], r0.v[0], r0.f[0]);
     if constexpr (sizeof(T) == 8)
         kb = __double_as_longlong((double)r0.v[0]) == 0 ? 0u : kb;
@@ -225,13 +236,28 @@ __device__ __forceinline__ double forward_line(T *p, At at, int n, double c1, co
     for (int j = 1; j < kBatch; ++j)
         if (j < n)
             row(r0.q[j], r0.v[j], r0.f[j]);
-    if (pairs > 0) {
-        request(2 * kBatch, r0);
-        for (int k = kBatch; k < end; k += 2 * kBatch) {
+    if (early > 0) {
+        request(2 * kBatch, r0, true);
+        for (int k = kBatch; k < same; k += 2 * kBatch) {
             batch(r1);
-            request(min(k + 2 * kBatch, end - kBatch), r1);
+            request(min(k + 2 * kBatch, same - kBatch), r1, true);
             batch(r0);
-            request(min(k + 3 * kBatch, end - kBatch), r0);
+            request(min(k + 3 * kBatch, same - kBatch), r0, true);
+        }
+    }
+    if (late > 0) {
+        const FwdRow<T> d = f[same];
+        request(same, r1, false);
+        request(same + kBatch, r0, false);
+        for (int k = same; k < end; k += 2 * kBatch) {
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j)
+                row(r1.q[j], r1.v[j], d);
+            request(min(k + 2 * kBatch, end - kBatch), r1, false);
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j)
+                row(r0.q[j], r0.v[j], d);
+            request(min(k + 3 * kBatch, end - kBatch), r0, false);
         }
     }
     if (end < n) {
@@ -246,9 +272,10 @@ __device__ __forceinline__ double forward_line(T *p, At at, int n, double c1, co
 }
 
 // Back substitution of the same line from its last row's value xv: rows n-2 .. 0 go to out(k, x),
-// in that order (k is wave-uniform).
+// in that order (k is wave-uniform).  Settled rows go in longer batches: two operations a row, a
+// batch of four would be shorter than the latency of its requests.
 template <class T, int kBatch, class At, class Out>
-__device__ __forceinline__ void back_line(const T *p, At at, int n, double xv, const double *c, Out out)
+__device__ __forceinline__ void back_line(const T *p, At at, int n, int settled, double xv, const double *c, Out out)
 {
     struct {
         T v[kBatch];
@@ -288,17 +315,51 @@ __device__ __forceinline__ void back_line(const T *p, At at, int n, double xv, c
             xv = fma(-r1.c[j], xv, (double)r1.v[j]);
             out(full + kBatch + j, xv);
         }
-    if (full > 0)
-        request(full - kBatch, r1);
 #pragma unroll
     for (int j = kBatch - 1; j >= 0; --j)
         if (full + j < n - 1) {
             xv = fma(-r0.c[j], xv, (double)r0.v[j]);
             out(full + j, xv);
         }
-    if (full > 0)
-        request(full - 2 * kBatch, r0);
-    for (int k = full - 2 * kBatch; k >= 0; k -= 2 * kBatch) {
+    // pairs of long batches while all their rows are settled
+    constexpr int kLong = 2 * kBatch;
+    const int late = max(full - settled, 0) / (2 * kLong), low = full - late * 2 * kLong;
+    if (late > 0) {
+        const double cs = c[full - 1];
+        T l0[kLong], l1[kLong];
+        auto ask = [&](int k, T *l) {
+#pragma unroll
+            for (int h = 0; h < kLong; h += kBatch) {
+                const T *q = p + at(k + h);
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) {
+                    l[h + j] = *q;
+                    q += at.step();
+                }
+            }
+            asm volatile("" ::: "memory");
+        };
+        auto go = [&](int k, const T *l) {
+#pragma unroll
+            for (int j = kLong - 1; j >= 0; --j) {
+                xv = fma(-cs, xv, (double)l[j]);
+                out(k + j, xv);
+            }
+        };
+        ask(full - kLong, l1);
+        ask(full - 2 * kLong, l0);
+        for (int k = full - 2 * kLong; k >= low; k -= 2 * kLong) {
+            go(k + kLong, l1);
+            ask(max(k - kLong, 0), l1);
+            go(k, l0);
+            ask(max(k - 2 * kLong, 0), l0);
+        }
+    }
+    if (low > 0) {
+        request(low - kBatch, r1);
+        request(low - 2 * kBatch, r0);
+    }
+    for (int k = low - 2 * kBatch; k >= 0; k -= 2 * kBatch) {
         batch(k + kBatch, r1);
         request(max(k - kBatch, 0), r1);
         batch(k, r0);
@@ -539,6 +600,7 @@ __global__ __launch_bounds__(kMaxThreads, (plane_waves_per_simd<T, BIG>())) void
         const double c1 = as_ctab(D.c1)[s];
         const bool pairx = sizeof(T) == 4 || as_ctab(D.tab[0].nopair)[s] == 0.0;
         const bool pairy = sizeof(T) == 4 || as_ctab(D.tab[1].nopair)[s] == 0.0;
+        const int setx = (int)as_ctab(D.tab[0].settled)[s], sety = (int)as_ctab(D.tab[1].settled)[s];
         const bool act = active(D, s);
         const T dv = ((const __attribute__((address_space(4))) T *)D.dval)[s];
         const gmem<const T> fv = as_global(D.dface);  // per-voxel Dirichlet values
@@ -614,37 +676,37 @@ __global__ __launch_bounds__(kMaxThreads, (plane_waves_per_simd<T, BIG>())) void
                     lds_barrier();
                 }
                 unsigned key = 0u;
-                auto forward = [&](T *q, auto rows, int n, bool pair, const double *den) {
+                auto forward = [&](T *q, auto rows, int n, int settled, bool pair, const double *den) {
                     if constexpr (sizeof(T) == 4)
-                        return forward_line<T, kPair, B>(q, rows, n, c1, tf, nullptr, key);
+                        return forward_line<T, kPair, B>(q, rows, n, settled, c1, tf, nullptr, key);
                     else
-                        return exact ? forward_line<T, kTrue, B>(q, rows, n, c1, tf, as_ctab(den), key)
-                                     : pair ? forward_line<T, kPair, B>(q, rows, n, c1, tf, nullptr, key)
-                                            : forward_line<T, kCorr, B>(q, rows, n, c1, tf, nullptr, key);
+                        return exact ? forward_line<T, kTrue, B>(q, rows, n, settled, c1, tf, as_ctab(den), key)
+                                     : pair ? forward_line<T, kPair, B>(q, rows, n, settled, c1, tf, nullptr, key)
+                                            : forward_line<T, kCorr, B>(q, rows, n, settled, c1, tf, nullptr, key);
                 };
                 const Contiguous row;
                 // a line on a Dirichlet face is overwritten whole, whatever its numerators were
                 auto x_forward = [&]() {
                     const unsigned k0 = key;
-                    const double y = forward(P + lay(tid), row, nx, pairx, D.tab[0].den + (size_t)s * nx);
+                    const double y = forward(P + lay(tid), row, nx, setx, pairx, D.tab[0].den + (size_t)s * nx);
                     if (act && (tid == 0 || tid == ny - 1))
                         key = k0;
                     return y;
                 };
                 auto x_back = [&](double y) {
                     T *q = P + lay(tid);
-                    back_line<T, B>(q, row, nx, y, tc, [&](int k, double x) { q[k] = (T)x; });
+                    back_line<T, B>(q, row, nx, setx, y, tc, [&](int k, double x) { q[k] = (T)x; });
                 };
                 auto y_forward = [&]() {
                     const unsigned k0 = key;
-                    const double y = forward(P + tid, lay, ny, pairy, D.tab[1].den + (size_t)s * ny);
+                    const double y = forward(P + tid, lay, ny, sety, pairy, D.tab[1].den + (size_t)s * ny);
                     if (act && (tid == 0 || tid == nx - 1))
                         key = k0;
                     return y;
                 };
                 auto y_back = [&](double y) {
                     T *q = P + tid;
-                    back_line<T, B>(q, lay, ny, y, tc, [&](int k, double x) { q[lay(k)] = (T)x; });
+                    back_line<T, B>(q, lay, ny, sety, y, tc, [&](int k, double x) { q[lay(k)] = (T)x; });
                 };
                 double last = 0.0;
                 if constexpr (!YX) {
@@ -694,7 +756,7 @@ __global__ __launch_bounds__(kMaxThreads, (plane_waves_per_simd<T, BIG>())) void
                         const bool face = act && (tid == 0 || tid == nx - 1);
                         gmem<T> q = f + tid + (size_t)(ny - 1) * nx;  // rows are stored from the last to the first
                         store_result<T>(q, act ? dv : (T)last);
-                        back_line<T, B>(P + tid, lay, ny, last, tc, [&](int k, double x) {
+                        back_line<T, B>(P + tid, lay, ny, sety, last, tc, [&](int k, double x) {
                             q -= nx;
                             store_result<T>(q, face || (act && k == 0) ? dv : (T)x);
                         });
