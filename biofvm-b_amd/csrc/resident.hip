@@ -540,6 +540,11 @@ __global__ __launch_bounds__(kMaxThreads, (plane_waves_per_simd<T, BIG>())) void
                         q[0] = r[j].x;
                         q[1] = r[j].y;
                     }
+                // a launch over uneven members may have more solvers, and so fewer loaders, than this
+                // plane alone would: what their registers could not hold
+                const gmem<const T> src = as_global<const T>(D.field[parity] + ((size_t)s * D.nz + z) * nel);
+                for (int e = 2 * kLoads * ln + lid; e < nel; e += ln)
+                    P[at(e, D.nx, lay, inv)] = src[e];
             }
             lds_barrier();  // plane and first tables in LDS
             t += gridDim.x;
@@ -831,7 +836,9 @@ int launch_planes_class(Group *g, int c, bool yx, bool agents)
             lines = std::max(lines, std::max(d.nx, d.ny));
         }
     const int solvers = (lines + kWave - 1) / kWave * kWave;
-    const unsigned th = BIG ? kMaxThreads : (unsigned)(solvers + plane_loaders(el, plane_loads<T, BIG>()));
+    // (resident_class leaves each member a wavefront of loaders at least)
+    const unsigned th = BIG ? kMaxThreads
+                            : (unsigned)std::min<size_t>(solvers + plane_loaders(el, plane_loads<T, BIG>()), kMaxThreads);
     // as many workgroups as the CUs hold, each striding over the planes
     const int waves = 4 * plane_waves_per_simd<T, BIG>() / (int)(th / kWave);
     const long long percu = std::max(1, std::min(waves, (int)(kLdsBytes / lds)));

@@ -162,3 +162,28 @@ def test_batch_of_resident_and_other_members(precision):
             s.run(6)
             assert np.array_equal(g, s.download())
             s.close()
+
+
+@pytest.mark.parametrize("precision,shapes", [
+    ("fp64", [(240, 60, 5, 1), (133, 120, 6, 2), (60, 240, 3, 1)]),   # 256 solvers leave 256 loaders
+    ("fp64", [(200, 30, 5, 1), (95, 95, 6, 2), (30, 200, 3, 1)]),     # more threads than a workgroup
+    ("fp32", [(320, 70, 5, 1), (190, 190, 4, 2), (70, 320, 3, 1)])])
+def test_batch_of_long_and_large_planes(precision, shapes):
+    """Members of one size class, some with many lines, some with many values: the launch has the
+    solvers of the former and then too few loaders to hold the latter's planes in registers."""
+    from biofvmb import Batch
+    cases = [_case(sh, seed=60 + i) for i, sh in enumerate(shapes)]
+    b = Batch(shapes, cases[0].dx, precision)
+    for i, c in enumerate(cases):
+        b.set_coefficients(i, c.D, c.decay, c.dt)
+        b.set_dirichlet(i, *cf.effective_dirichlet(c))
+        b.upload(i, c.init)
+        b.set_agents(i, *orc.agent_tables(c))
+    b.run(3)
+    got = [b.download(i) for i in range(len(shapes))]
+    b.close()
+    for c, g in zip(cases, got):
+        s = _solver(c, precision, separate=True)
+        s.run(3)
+        assert np.array_equal(g, s.download())
+        s.close()
