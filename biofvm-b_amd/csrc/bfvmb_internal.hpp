@@ -35,8 +35,10 @@ enum Phase {
     kSweep0 = 1,                      // x, y, z tiles
     kBulk0 = 4,                       // bulk elements
     kPlane0 = 5,                      // planes in LDS, by class
-    kRest0 = kPlane0 + kClasses,      // agents, x, y tiles of the domains outside those
-    kPhases = kRest0 + 3
+    kRest0 = kPlane0 + kClasses,      // agents, x, y tiles of the domains outside those (agents and
+                                      // x: outside the strips too)
+    kStrip0 = kRest0 + 3,             // strips of rows in LDS
+    kPhases
 };
 
 // Per-axis Thomas tables, FP64 on both storage paths, [nsub][n].
@@ -65,11 +67,13 @@ struct DomainDesc {
     const int *xseg;             // agents: [x-sweep tiles per substrate + 1] first segment of
                                  // each tile of 64 rows (z*ny + y), or nullptr: no agents
     const int *zseg;             // agents: [nz + 1] first segment of each z plane, or nullptr: no agents
+    const int *sseg;             // agents: [strips + 1] first segment of each strip of rows, or nullptr
     const double *bulk_ts;       // bulk: [nsub][nz][ny][nx] target*supply (nullptr: none)
     const double *bulk_us;       // bulk: [nsub][nz][ny][nx] uptake+supply
     double dt;                   // time step frozen by set_coefficients
     int nseg, nact;
     int nx, ny, nz, nsub;
+    int strip;                   // rows (z*ny + y) of a strip in LDS, 0: rows do not fit
 };
 
 // Per-voxel Dirichlet values of a domain's six faces, in one array of the field's precision:
@@ -124,7 +128,10 @@ struct Domain {
     size_t seg_cap = 0, act_cap = 0;  // segments / agents the device arrays have room for
     int *xseg = nullptr;           // first segment of each x-sweep tile (rebuilt with the descriptors)
     int *zseg = nullptr;           // first segment of each z plane (likewise)
+    int *sseg = nullptr;           // first segment of each strip of rows (likewise)
     int plane_class = -1;          // LDS size class of its z planes, -1: they do not fit
+    int strip = 0;                 // rows of a strip in LDS (strip_rows)
+    bool strips = false;           // its x sweep goes by strips: planes do not fit, strips do
     std::vector<int> agent_order;  // sorted position -> index in the caller's agent list (after
                                    // moves: current once domain_agent_order has run)
     std::vector<long long> agent_off;  // device offset of each sorted agent's voxel, as set
@@ -178,7 +185,10 @@ struct Group {
 // field[cur] -> field[cur^1] for every domain, or for those not swept in LDS (rest)
 int launch_sweep(Group *g, int axis, bool rest = false);
 int launch_planes(Group *g, bool yx, bool agents);  // resident planes, in place on field[cur]
+int launch_strips(Group *g, bool agents);           // x sweep by strips, to field[cur ^ 1] (cur stays)
 void resident_class(const Group *g, Domain &d);
+int strip_rows(const Domain &d, size_t elem, size_t limit);
+bool strips_pay(const Group *g, const Domain &d, long long strips, long long before);
 int resident_lds_attributes(size_t bytes);
 int launch_sweep_x_agents(Group *g, bool rest = false);  // cell sources/sinks, then the x sweep, in one launch
 int launch_xseg(Group *g, const Domain &d);  // xseg from the domain's segment list

@@ -317,6 +317,11 @@ int launch_xseg(Group *g, const Domain &d)
                        d.nx, nrows, kWave, ntiles, d.xseg);
     hipLaunchKernelGGL(k_xseg, dim3((unsigned)((d.nz + 1 + 255) / 256)), dim3(256), 0, g->stream, d.seg_off, d.nseg,
                        d.nx, nrows, d.ny, d.nz, d.zseg);
+    if (d.strip > 0) {
+        const int strips = (int)((nrows + d.strip - 1) / d.strip);
+        hipLaunchKernelGGL(k_xseg, dim3((unsigned)((strips + 1 + 255) / 256)), dim3(256), 0, g->stream, d.seg_off, d.nseg,
+                           d.nx, nrows, d.strip, strips, d.sseg);
+    }
     return hip_check(g, hipGetLastError(), "agent tile index launch");
 }
 

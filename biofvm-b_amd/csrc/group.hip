@@ -108,6 +108,8 @@ std::vector<DomainDesc<T>> build_descs(Group *g)
         e.t2 = d.t2;
         e.xseg = d.nseg > 0 ? d.xseg : nullptr;
         e.zseg = d.nseg > 0 ? d.zseg : nullptr;
+        e.sseg = d.nseg > 0 ? d.sseg : nullptr;
+        e.strip = d.strip;
         e.bulk_ts = d.bulk;
         e.bulk_us = d.bulk ? d.bulk + d.nvox * d.nsub : nullptr;
         e.dt = d.dt;
@@ -149,6 +151,8 @@ int sync_descriptors(Group *g)
         resident_class(g, d);
         if (d.plane_class >= 0 && g->prefix[kPlane0 + d.plane_class][i] + (long long)d.nz * d.nsub > (1 << 30))
             d.plane_class = -1;  // a launch counts its planes in int
+        const long long strips = d.strip ? ((d.ny * (long long)d.nz + d.strip - 1) / d.strip) * d.nsub : 0;
+        d.strips = d.plane_class < 0 && strips_pay(g, d, strips, g->prefix[kStrip0][i]);
         long long work[kPhases] = {};
         work[kAgents0] = (long long)d.nseg * d.nsub;
         work[kSweep0] = (long long)((d.ny * (long long)d.nz + kWave - 1) / kWave) * d.nsub;
@@ -158,8 +162,10 @@ int sync_descriptors(Group *g)
         if (d.plane_class >= 0)
             work[kPlane0 + d.plane_class] = (long long)d.nz * d.nsub;
         else
-            for (int p = 0; p < 3; ++p)
+            for (int p = d.strips ? 2 : 0; p < 3; ++p)
                 work[kRest0 + p] = work[p];
+        if (d.strips)
+            work[kStrip0] = strips;
         for (int p = 0; p < kPhases; ++p)
             g->prefix[p][i + 1] = g->prefix[p][i] + work[p];
     }
@@ -264,6 +270,9 @@ int group_init(Group *g, int ndom, const int *nx, const int *ny, const int *nz, 
             (rc = hip_check(g, hipMalloc((void **)&d.xseg, ((d.ny * (size_t)d.nz + kWave - 1) / kWave + 1) * sizeof(int)),
                             "agent tile index")) ||
             (rc = hip_check(g, hipMalloc((void **)&d.zseg, (d.nz + 1) * sizeof(int)), "agent plane index")) ||
+            (d.strip = strip_rows(d, g->elem, g->max_lds_per_block),
+             rc = hip_check(g, hipMalloc((void **)&d.sseg, (d.strip ? (d.ny * (size_t)d.nz + d.strip - 1) / d.strip + 1 : 1) *
+                                                               sizeof(int)), "agent strip index")) ||
             (rc = hip_check(g, hipMemsetAsync(d.field[0], 0, bytes, g->stream), "zero field")) ||
             (rc = upload_dirichlet(g, d)))
             return rc;
@@ -289,6 +298,7 @@ void group_free(Group *g)
         (void)hipFree(d.d_dact);
         (void)hipFree(d.xseg);
         (void)hipFree(d.zseg);
+        (void)hipFree(d.sseg);
         (void)hipFree(d.d_dface);
     }
     adjoint_free(g);
@@ -680,6 +690,26 @@ static int launch_agents_and_x(Group *g, bool rest = false)
     return rc ? rc : launch_sweep(g, 0, rest);
 }
 
+// The x sweep (and the cell sources and sinks before it) of every domain, or (rest) of those
+// whose planes are not swept in LDS: by strips in LDS where rows fit, by lod.hip's kernel elsewhere.
+static int launch_x(Group *g, bool agents, bool rest)
+{
+    int rc;
+    if (rest) {
+        if ((rc = launch_strips(g, agents)))
+            return rc;
+        if (g->prefix[kRest0 + 1].back() == 0) {
+            g->cur ^= 1;
+            return BFVMB_OK;
+        }
+    }
+    // FP64: the cell sources and sinks run inside the x sweep, tile by tile, before it
+    // reads each tile (results identical to a separate pass; one launch fewer), unless a
+    // tile is dense (kFuseMaxSegsPerTile).  FP32 keeps the separate pass: its x sweep runs
+    // one wavefront per SIMD, which leaves no other wavefront to cover the update's latency.
+    return agents ? launch_agents_and_x(g, rest) : launch_sweep(g, 0, rest);
+}
+
 int launch_step(Group *g, bool with_agents)
 {
     int rc;
@@ -688,13 +718,8 @@ int launch_step(Group *g, bool with_agents)
     const bool rest = g->planes;
     if (rest && (rc = launch_planes(g, false, with_agents)))
         return rc;
-    // FP64: the cell sources and sinks run inside the x sweep, tile by tile, before it
-    // reads each tile (results identical to a separate pass; one launch fewer), unless a
-    // tile is dense (kFuseMaxSegsPerTile).  FP32 keeps the separate pass: its x sweep runs
-    // one wavefront per SIMD, which leaves no other wavefront to cover the update's latency.
-    if ((!rest || g->prefix[kRest0 + 1].back() > 0) &&
-        ((rc = with_agents ? launch_agents_and_x(g, rest) : launch_sweep(g, 0, rest)) ||
-         (rc = launch_sweep(g, 1, rest))))
+    if ((!rest || g->prefix[kRest0 + 2].back() > 0) &&
+        ((rc = launch_x(g, with_agents, rest)) || (rc = launch_sweep(g, 1, rest))))
         return rc;
     return launch_sweep(g, 2);
 }
@@ -707,8 +732,8 @@ int launch_step_adjoint(Group *g)
     const bool rest = g->planes;
     if (rest && (rc = launch_planes(g, true, false)))
         return rc;
-    if (!rest || g->prefix[kRest0 + 1].back() > 0)
-        if ((rc = launch_sweep(g, 1, rest)) || (rc = launch_sweep(g, 0, rest)))
+    if (!rest || g->prefix[kRest0 + 2].back() > 0)
+        if ((rc = launch_sweep(g, 1, rest)) || (rc = launch_x(g, false, rest)))
             return rc;
     return BFVMB_OK;
 }
@@ -873,14 +898,14 @@ int group_autotune(Group *g, int reps, int *chosen)
             chosen[3 * axis + 2] = (int)(best * 1000.f / reps);  // microseconds per launch
         }
     }
-    // planes in LDS (both sweeps) against the separate sweeps at those shapes
+    // planes and strips in LDS against the separate sweeps at those shapes
     const bool planes = g->planes;
     bool any = false;
     for (const Domain &d : g->doms)
-        any = any || d.plane_class >= 0;
+        any = any || d.plane_class >= 0 || d.strips;
     auto once = [&]() -> int {
         int e = launch_planes(g, false, false);
-        if (!e && g->prefix[kRest0 + 1].back() > 0 && !(e = launch_sweep(g, 0, true)))
+        if (!e && g->prefix[kRest0 + 2].back() > 0 && !(e = launch_x(g, false, true)))
             e = launch_sweep(g, 1, true);
         return e;
     };

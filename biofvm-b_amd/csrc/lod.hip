@@ -1196,8 +1196,8 @@ int launch_sweep_t(Group *g, int axis, bool agents, bool rest)
     if (rc)
         return rc;
     const int ndom = (int)g->doms.size();
-    // rest: only the domains whose planes are not swept in LDS
-    auto skip = [&](const Domain &d) { return rest && d.plane_class >= 0; };
+    // rest: only the domains whose planes (x: or strips) are not swept in LDS
+    auto skip = [&](const Domain &d) { return rest && (d.plane_class >= 0 || (axis == 0 && d.strips)); };
     const Shape sh = shape_of(g, axis);
     XVariant xv = x_variant<T>(sh.bpc, axis == 0 ? sh.ring : 0);
     if (axis == 0 && xv.tl) {

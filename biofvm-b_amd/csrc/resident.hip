@@ -1,4 +1,5 @@
-// resident.hip -- the x and y sweeps of whole z planes held in LDS.
+// resident.hip -- the x and y sweeps of whole z planes held in LDS, and the FP64 x sweep of strips of
+// rows where planes do not fit (k_strip).
 //
 // The kernels of lod.hip stream a line through a ring of rows and keep of it what fits on chip;
 // they are made for lines and fields far larger than a CU's storage.  Where a z plane of one
@@ -791,6 +792,290 @@ __global__ __launch_bounds__(kMaxThreads, (plane_waves_per_simd<T, BIG>())) void
     }
 }
 
+// ---- strips: the FP64 x sweep of rows in LDS, for planes that do not fit there
+
+constexpr int kStripLoads = 31;  // pairs per loading thread
+
+// One strip: `rows` consecutive rows (z*ny + y) of one substrate from row r0, strip i of it.
+template <class T>
+struct Strip {
+    const DomainDesc<T> *D;
+    int di, s, i, r0, rows;
+};
+
+template <class T>
+__device__ __forceinline__ Strip<T> locate_strip(const DomainDesc<T> *descs, const long long *prefix, int ndom, int t)
+{
+    Strip<T> p;
+    long long lt = t;
+    p.di = 0;
+    if (ndom > 1) {
+        p.di = __builtin_amdgcn_readfirstlane(find_domain(prefix, ndom, lt));
+        lt -= prefix[p.di];
+    }
+    p.D = descs + p.di;
+    const unsigned R = (unsigned)p.D->strip, all = (unsigned)p.D->ny * (unsigned)p.D->nz, n = (all + R - 1) / R;
+    p.s = __builtin_amdgcn_readfirstlane((int)((unsigned)lt / n));
+    p.i = __builtin_amdgcn_readfirstlane((int)((unsigned)lt - (unsigned)p.s * n));
+    p.r0 = p.i * (int)R;
+    p.rows = (int)min(R, all - (unsigned)p.r0);
+    return p;
+}
+
+// What bounds it: the solvers need 68 + 36 clocks per column forward and back (64 rows of 256: 10 us),
+// then 128 KB go out and the next strip goes in, during which no row is solved; a CU has LDS for one
+// strip of such rows, so the memory system idles in the solve and queues in between (256^3 x 4 FP64:
+// 0.31 ms, 3.5 TB/s).  It still beats lod.hip's x sweep (0.37 ms) in FP64, which reads most of each line
+// twice.  Tried: results out in column segments during back substitution (256^3 x 4 783 -> 834 us per
+// step), a staggered start of the workgroups and contiguous strips per XCD (no change).
+//
+// Workgroups stride over the strips; the first `solvers` threads sweep, a row per lane, the other
+// wavefronts hold the next strip in registers meanwhile, as k_plane's do.  Reads field[parity],
+// writes field[parity ^ 1].  AG: the cell sources and sinks first, on the strip in LDS; the loaders
+// also fetch the next strip's (one voxel each; what a denser strip has more is fetched when applied).
+// NT: non-temporal loads and stores.
+template <class T, bool AG, bool NT>
+__global__ __launch_bounds__(kMaxThreads, 2) void k_strip(const DomainDesc<T> *__restrict__ descs,
+                                                          const long long *__restrict__ prefix, int ndom, int strips,
+                                                          int solvers, int parity)
+{
+    constexpr int kLoads = kStripLoads, B = 4;
+    typedef typename PairOf<T>::type Pair;
+    extern __shared__ unsigned char smem[];
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int wave_first = __builtin_amdgcn_readfirstlane(tid);
+
+    auto lds_tables = [&]() { return reinterpret_cast<FwdRow<T> *>(smem); };
+    auto lds_factors = [&](const DomainDesc<T> &D) { return reinterpret_cast<double *>(lds_tables() + D.nx); };
+    auto lds_strip = [&](const DomainDesc<T> &D) { return reinterpret_cast<T *>(lds_factors(D) + D.nx); };
+    // LDS index of the strip's element e: rows lie nx | 1 apart
+    auto at = [](int e, int nx, unsigned inv) { return nx & 1 ? e : e + quot(e, inv); };
+    auto source = [&](const Strip<T> &p, int par) {
+        return as_global(p.D->field[par] + ((size_t)p.s * ((size_t)p.D->ny * p.D->nz) + p.r0) * p.D->nx);
+    };
+    auto copy_out = [&](const Strip<T> &p) {
+        const int nx = p.D->nx, n = p.rows * nx;
+        const unsigned inv = quot_inv(nx);
+        const T *P = lds_strip(*p.D);
+        const gmem<T> f = source(p, parity ^ 1);
+        int e = 2 * tid;
+        for (; e < n - 1; e += 2 * nt) {
+            const T *q = P + at(e, nx, inv);
+            Pair v;
+            v.x = q[0];
+            v.y = q[1];
+            if constexpr (NT)
+                __builtin_nontemporal_store(v, (gmem<Pair>)(f + (unsigned)e));
+            else
+                *(gmem<Pair>)(f + (unsigned)e) = v;
+        }
+        if (e == n - 1)
+            f[e] = P[at(e, nx, inv)];
+    };
+    auto update = [](T *q, const gmem<const double> a1, const gmem<const double> a2, int b0, int b1) {
+        double v = (double)*q;
+        for (int a = b0; a < b1; ++a) {
+            v = v + a1[a];
+            v = v / a2[a];
+        }
+        *q = (T)v;
+    };
+
+    if (wave_first >= solvers) {
+        // ------------------------------------------------------------------ loading wavefronts
+        const int lid = tid - solvers, ln = nt - solvers;
+        Pair r[kLoads];
+        auto first = [&](int j, int n) { return min(2 * (lid + j * ln), n - 2); };
+        int ag_e = -1, ag_b0 = 0, ag_b1 = 0;  // this thread's voxel with agents in the next strip
+        double ag_1 = 0.0, ag_2 = 1.0;
+        auto request = [&](const Strip<T> &p) {
+            const DomainDesc<T> &D = *p.D;
+            if (AG && D.sseg != nullptr) {
+                const auto ss = (const __attribute__((address_space(4))) int *)D.sseg;
+                const int k = ss[p.i] + lid;
+                ag_e = -1;
+                if (k < ss[p.i + 1]) {
+                    ag_e = (int)(as_global(D.seg_off)[k] - (long long)p.r0 * D.nx);
+                    ag_b0 = as_global(D.seg_start)[k];
+                    ag_b1 = as_global(D.seg_start)[k + 1];
+                    ag_1 = as_global(D.t1 + (size_t)p.s * D.nact)[ag_b0];
+                    ag_2 = as_global(D.t2 + (size_t)p.s * D.nact)[ag_b0];
+                }
+            }
+            const int n = p.rows * D.nx;
+            const gmem<const T> src = source(p, parity);
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+                if (2 * j * ln < n)
+                    if constexpr (NT)
+                        r[j] = __builtin_nontemporal_load((gmem<const Pair>)(src + (unsigned)first(j, n)));
+                    else
+                        r[j] = *(gmem<const Pair>)(src + (unsigned)first(j, n));
+        };
+        int t = blockIdx.x;
+        Strip<T> p = locate_strip(descs, prefix, ndom, t);
+        request(p);
+        for (;;) {
+            const Strip<T> now = p;
+            const DomainDesc<T> &D = *now.D;
+            T *P = lds_strip(D);
+            const int nx = D.nx, n = now.rows * nx;
+            const unsigned inv = quot_inv(nx);
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+                if (2 * j * ln < n) {
+                    int e = first(j, n);
+                    asm("" : "+v"(e));  // so many LDS addresses are cheaper to form than to keep
+                    T *q = P + at(e, nx, inv);  // a pair stays in its row where rows are padded (nx even)
+                    q[0] = r[j].x;
+                    q[1] = r[j].y;
+                }
+            lds_barrier();  // strip and tables in LDS
+            if (AG && D.sseg != nullptr) {
+                const gmem<const double> a1 = as_global<const double>(D.t1 + (size_t)now.s * D.nact);
+                const gmem<const double> a2 = as_global<const double>(D.t2 + (size_t)now.s * D.nact);
+                if (ag_e >= 0) {
+                    T *q = P + at(ag_e, nx, inv);
+                    double v = ((double)*q + ag_1) / ag_2;
+                    for (int a = ag_b0 + 1; a < ag_b1; ++a) {
+                        v = v + a1[a];
+                        v = v / a2[a];
+                    }
+                    *q = (T)v;
+                }
+                const auto ss = (const __attribute__((address_space(4))) int *)D.sseg;
+                for (int k = ss[now.i] + lid + ln; k < ss[now.i + 1]; k += ln)
+                    update(P + at((int)(as_global(D.seg_off)[k] - (long long)now.r0 * nx), nx, inv), a1, a2,
+                           as_global(D.seg_start)[k], as_global(D.seg_start)[k + 1]);
+                lds_barrier();  // agents
+            }
+            t += gridDim.x;
+            if (t < strips) {
+                p = locate_strip(descs, prefix, ndom, t);
+                request(p);
+            }
+            lds_barrier();  // solved
+            copy_out(now);
+            if (t >= strips)
+                return;
+            lds_barrier();  // the strip's LDS is free
+        }
+    }
+
+    // ---------------------------------------------------------------------- solving wavefronts
+    int t = blockIdx.x, di_had = -1, s_had = -1;
+    for (;;) {
+        const Strip<T> p = locate_strip(descs, prefix, ndom, t);
+        const DomainDesc<T> &D = *p.D;
+        const int s = p.s, nx = D.nx, ny = D.ny, nz = D.nz;
+        const unsigned inv = quot_inv(nx);
+        const double c1 = as_ctab(D.c1)[s];
+        const bool pair = as_ctab(D.tab[0].nopair)[s] == 0.0;
+        const int settled = (int)as_ctab(D.tab[0].settled)[s];
+        const bool act = __builtin_amdgcn_readfirstlane((int)as_global(D.dact)[s]) != 0;
+        const T dv = ((const __attribute__((address_space(4))) T *)D.dval)[s];
+        const gmem<const T> fv = as_global(D.dface);  // per-voxel Dirichlet values
+        const bool voxels = D.dface != nullptr;
+        FwdRow<T> *tf = lds_tables();
+        double *tc = lds_factors(D);
+        T *P = lds_strip(D);
+        if (p.di != di_had || s != s_had) {
+            for (int k = tid; k < nx; k += solvers) {
+                FwdRow<T> f;
+                double c;
+                load_row<T>(D.tab[0], (size_t)s * nx, nx, pair, k, f, c);
+                tf[k] = f;
+                tc[k] = c;
+            }
+            di_had = p.di;
+            s_had = s;
+        }
+        const bool mine = tid < p.rows;
+        const int row = p.r0 + (mine ? tid : 0), z = row / ny, y = row - z * ny;
+        const bool face = act && (y == 0 || y == ny - 1 || z == 0 || z == nz - 1);
+        T *q = P + (mine ? tid : 0) * (nx | 1);
+        auto ends = [&]() {  // the row's voxels on the x faces
+            if (act && mine) {
+                q[0] = voxels ? fv[face_x(ny, nz, D.nsub, 0, s, y, z)] : dv;
+                q[nx - 1] = voxels ? fv[face_x(ny, nz, D.nsub, 1, s, y, z)] : dv;
+            }
+        };
+        lds_barrier();  // strip and tables in LDS
+        if (AG && D.sseg != nullptr)
+            lds_barrier();  // agents
+        ends();
+        double last = 0.0;
+        unsigned key = 0u;
+        const Contiguous cols;
+        auto forward = [&](auto div) {
+            if (mine)
+                last = forward_line<T, decltype(div)::value, B>(q, cols, nx, settled, c1, tf,
+                                                                as_ctab(D.tab[0].den + (size_t)s * nx), key);
+        };
+        if (pair)
+            forward(std::integral_constant<int, kPair>());
+        else
+            forward(std::integral_constant<int, kCorr>());
+        // a numerator outside the fast divisions' range: this wavefront's rows again from
+        // memory (which still holds them) with true divisions.  A row on a face is overwritten.
+        if (__ballot(mine && !face && key >= kKeyBad) != 0) {
+            const int l0 = wave_first / kWave * kWave, l1 = min(l0 + kWave, p.rows), lane = tid - l0;
+            const gmem<const T> src = source(p, parity);
+            for (int e = l0 * nx + lane; e < l1 * nx; e += kWave)
+                P[at(e, nx, inv)] = src[e];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+            if (AG && D.sseg != nullptr) {
+                const auto ss = (const __attribute__((address_space(4))) int *)D.sseg;
+                for (int k = ss[p.i] + lane; k < ss[p.i + 1]; k += kWave) {
+                    const int e = (int)(as_global(D.seg_off)[k] - (long long)p.r0 * nx);
+                    if (e >= l0 * nx && e < l1 * nx)
+                        update(P + at(e, nx, inv), as_global<const double>(D.t1 + (size_t)s * D.nact),
+                               as_global<const double>(D.t2 + (size_t)s * D.nact), as_global(D.seg_start)[k],
+                               as_global(D.seg_start)[k + 1]);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+            }
+            ends();
+            forward(std::integral_constant<int, kTrue>());
+        }
+        if (mine) {
+            q[nx - 1] = (T)last;
+            back_line<T, B>(q, cols, nx, settled, last, tc, [&](int k, double x) { q[k] = (T)x; });
+        }
+        ends();
+        unsigned long long faces = __ballot(mine && face);
+        while (faces != 0) {  // whole rows on the y and z faces
+            const int l = __builtin_amdgcn_readfirstlane(__ffsll((long long)faces) - 1);
+            faces &= faces - 1;
+            const int fl = wave_first / kWave * kWave + l, fr = p.r0 + fl, fz = fr / ny, fy = fr - fz * ny;
+            const bool zf = fz == 0 || fz == nz - 1;
+            const size_t base = !voxels ? 0
+                                : zf    ? face_z(nx, ny, nz, D.nsub, fz == 0 ? 0 : 1, s, 0, fy)
+                                        : face_y(nx, ny, nz, D.nsub, fy == 0 ? 0 : 1, s, 0, fz);
+            for (int x = tid % kWave; x < nx; x += kWave)
+                P[fl * (nx | 1) + x] = voxels ? fv[base + x] : dv;
+        }
+        lds_barrier();  // solved
+        copy_out(p);
+        t += gridDim.x;
+        if (t >= strips)
+            return;
+        lds_barrier();  // the strip's LDS is free
+    }
+}
+
+size_t strip_bytes(int nx, int rows, size_t elem)
+{
+    return (size_t)nx * (elem == 8 ? table_bytes<double>() : table_bytes<float>()) +
+           ((size_t)rows * (nx | 1) + 1) * elem;
+}
+
+// Fields up to this size stay in the 256 MB memory-side cache for the y sweep; larger ones are read
+// and written non-temporally (250 x 230 x 210 x 2 FP64, 193 MB: 322 -> 299 us per step, 256^3 x 4 806 ->
+// 783; 160^3 x 4, 131 MB: 190 -> 200).
+constexpr size_t kStripCached = 160u << 20;
+constexpr size_t kStripSmall = 192u << 20;  // "large fields" of strips_pay
+
 template <bool SKEW>
 size_t plane_bytes(const Domain &d, size_t elem)
 {
@@ -891,6 +1176,67 @@ hipError_t attributes_all(int bytes)
 
 }  // namespace
 
+int strip_rows(const Domain &d, size_t elem, size_t limit)
+{
+    limit = std::min(limit, kLdsBytes);
+    const size_t tables = strip_bytes(d.nx, 0, elem), row = (size_t)(d.nx | 1) * elem;
+    const size_t loads = 2 * (size_t)kStripLoads;
+    if (elem != 8 || d.nx < 2 || tables + row > limit)
+        return 0;
+    // two workgroups of 64 rows per CU, or one of as many rows as fit, 128 at most
+    if (tables + kWave * row <= limit / 2 && (size_t)d.nx * kWave <= loads * (kMaxThreads / 2 - kWave))
+        return kWave;
+    size_t r = std::min<size_t>((limit - tables) / row, 2 * kWave);
+    r = std::min(r, loads * (kMaxThreads - 2 * kWave) / d.nx);
+    return r >= 32 ? (int)r : 0;
+}
+
+// Whether its x sweep goes by `strips` strips, `before` of other domains in the launch.  FP64 only:
+// lod.hip's FP32 kernel holds whole lines on chip and streams better (400 x 400 x 40, three simulations on
+// a stream each: 49 against 57 us per step).  FP64 where 32 rows fit (28 rows of 640 columns: 1597 ->
+// 1685), except large fields of rows of whole 128-byte lines below 320 columns, which lod.hip stores
+// non-temporally and reads again least.  Microseconds per step of one simulation, lod.hip's x sweep ->
+// strips (in brackets: of three in turn, on a stream each): 250 x 230 x 210 x 2 400 -> 297 (351 -> 286),
+// 300^3 x 2 829 -> 677 (756 -> 638), 200^3 x 2 208 -> 198 (203 -> 183), 192^3 x 3 280 -> 245 (245 -> 223),
+// 160^3 x 4 217 -> 185 (168 -> 169), 400^3 x 2 1552 -> 1478 (1331 -> 1306), 512 x 512 x 128 480 -> 455
+// (385 -> 386); 256^3 x 4, with its agents, 862 -> 815, but (696 -> 715).
+bool strips_pay(const Group *g, const Domain &d, long long strips, long long before)
+{
+    if (g->elem != 8 || strips == 0 || before + strips > (1 << 30))
+        return false;
+    return d.nx * sizeof(double) % 128 != 0 || d.nx >= 320 || d.nvox * d.nsub * sizeof(double) <= kStripSmall;
+}
+
+int launch_strips(Group *g, bool agents)
+{
+    int rc = sync_descriptors(g);
+    if (rc)
+        return rc;
+    const int ndom = (int)g->doms.size();
+    const long long strips = g->prefix[kStrip0][ndom];
+    if (strips == 0)
+        return BFVMB_OK;
+    size_t lds = 0, bytes = 0;
+    int rows = 0;
+    for (const Domain &d : g->doms)
+        if (d.strips) {
+            lds = std::max(lds, strip_bytes(d.nx, d.strip, sizeof(double)));
+            bytes += d.nvox * d.nsub * sizeof(double);
+            rows = std::max(rows, d.strip);
+        }
+    const int solvers = (rows + kWave - 1) / kWave * kWave;
+    const bool two = 2 * lds <= kLdsBytes;  // two workgroups per CU share its wavefronts
+    const unsigned th = two ? kMaxThreads / 2 : kMaxThreads;
+    const unsigned grid = (unsigned)std::min<long long>(strips, (two ? 2 : 1) * std::max(g->cu_count, 1));
+    const DomainDesc<double> *d = static_cast<const DomainDesc<double> *>(g->d_desc);
+    const long long *pre = g->d_prefix + (size_t)kStrip0 * (ndom + 1);
+    const bool nt = bytes > kStripCached;
+    const auto k = agents ? (nt ? k_strip<double, true, true> : k_strip<double, true, false>)
+                          : (nt ? k_strip<double, false, true> : k_strip<double, false, false>);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(th), lds, g->stream, d, pre, ndom, (int)strips, solvers, g->cur);
+    return hip_check(g, hipGetLastError(), "strip launch");
+}
+
 void resident_class(const Group *g, Domain &d)
 {
     const size_t limit = std::min(kLdsBytes, g->max_lds_per_block), el = (size_t)d.nx * d.ny;
@@ -919,6 +1265,10 @@ int resident_lds_attributes(size_t lds_bytes)
 {
     const int bytes = (int)std::min(lds_bytes, kLdsBytes);
     hipError_t e = attributes_all<double>(bytes);
+    const void *strip[4] = {(const void *)k_strip<double, false, false>, (const void *)k_strip<double, false, true>,
+                            (const void *)k_strip<double, true, false>, (const void *)k_strip<double, true, true>};
+    for (int i = 0; i < 4 && e == hipSuccess; ++i)
+        e = hipFuncSetAttribute(strip[i], hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e == hipSuccess)
         e = attributes_all<float>(bytes);
     return (int)e;

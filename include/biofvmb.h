@@ -167,7 +167,8 @@ int bfvmb_simulate_diffusion_decay(bfvmb_ctx *ctx, int nsteps);
 /* nsteps of the demo time loop (complete_diffusion_demo.cpp:489-493): per step, cell
  * sources/sinks then one LOD step (preceded by the bulk update when bulk rates are set).
  * Where a z plane of a substrate fits into a CU's LDS (FP64 up to about 139 x 139, FP32
- * 200 x 200), sources/sinks and the x and y sweeps are one launch over planes.  Elsewhere, in FP64 the sources/sinks run inside the x sweep's launch unless some x-sweep tile (64
+ * 200 x 200), sources/sinks and the x and y sweeps are one launch over planes; where only rows
+ * do (FP64, most fields up to 512 columns), sources/sinks and the x sweep are.  Elsewhere, in FP64 the sources/sinks run inside the x sweep's launch unless some x-sweep tile (64
  * rows y,z) holds more than 3072 occupied voxels; either way the results are those of the
  * two separate calls, bit for bit. */
 int bfvmb_run(bfvmb_ctx *ctx, int nsteps);
