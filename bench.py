@@ -73,8 +73,8 @@ def time_steps(s, torch, steps, warmup):
 
 def time_phases(s, torch, count=10):
     """Kernel times inside the step: `count` steps launched kernel by kernel as `run()` launches
-    them (FP64: the x sweep with the cell sources and sinks in its launch, then the y and z
-    sweeps; FP32: the agent kernel, then the three sweeps) with a HIP event on the library's
+    them where planes do not fit into LDS (FP64: the x sweep, by strips in LDS where those fit,
+    with the cell sources and sinks in its launch, then the y and z sweeps; FP32: the agent kernel, then the three sweeps) with a HIP event on the library's
     stream between consecutive kernels, so each kernel runs after the kernel it follows in a
     step (a sweep launched right after another launch of itself runs 3-7% faster than in the
     step).  Returns ms per launch of each kernel and "step", their sum."""
@@ -277,11 +277,11 @@ def traffic_record(dom):
     if not os.path.exists(tpath):
         return None, None
     rec = json.load(open(tpath))
-    src = os.path.join(ROOT, "biofvm-b_amd", "csrc", "lod.hip")
-    cur = hashlib.sha256(open(src, "rb").read()).hexdigest()
-    meta = {"profile": "profiles/traffic_400cube_fp64.json", "lod_hip_sha256": rec.get("lod_hip_sha256"),
-            "current_lod_hip_sha256": cur, "commit": rec.get("commit")}
-    if rec.get("lod_hip_sha256") != cur:
+    csrc = os.path.join(ROOT, "biofvm-b_amd", "csrc")
+    cur = hashlib.sha256(b"".join(open(os.path.join(csrc, f), "rb").read() for f in ("lod.hip", "resident.hip"))).hexdigest()
+    meta = {"profile": "profiles/traffic_400cube_fp64.json", "sweep_source_sha256": rec.get("sweep_source_sha256"),
+            "current_sweep_source_sha256": cur, "commit": rec.get("commit")}
+    if rec.get("sweep_source_sha256") != cur:
         meta["stale"] = True
         return None, meta
     return rec.get("bytes_per_launch", {}).get(dom), meta

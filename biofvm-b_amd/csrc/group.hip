@@ -803,8 +803,18 @@ int group_launch_phase(Group *g, int phase, int count)
             if (!d.have_coef)
                 return set_error(g, BFVMB_ERR_STATE, "set_coefficients has not been called for every domain");
     g->epoch++;
+    int rc0 = sync_descriptors(g);
+    if (rc0)
+        return rc0;
+    bool strips = false, planes = false;
+    for (const Domain &d : g->doms) {
+        strips = strips || d.strips;
+        planes = planes || d.plane_class >= 0;
+    }
     for (int i = 0; i < count; ++i) {
-        int rc = phase == 0 ? launch_agents(g) : phase == 4 ? launch_agents_and_x(g) : launch_sweep(g, phase - 1);
+        int rc = phase == 0   ? launch_agents(g)
+                 : phase == 4 ? launch_x(g, true, g->planes && strips && !planes)
+                              : launch_sweep(g, phase - 1);
         if (rc)
             return rc;
     }

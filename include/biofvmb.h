@@ -183,7 +183,7 @@ int bfvmb_sync(bfvmb_ctx *ctx);
 
 /* One kernel of the step, for measurement: phase 0 = sources/sinks, 1 = x, 2 = y, 3 = z
  * sweep, 4 = sources/sinks and x sweep as bfvmb_run launches them where it sweeps x and y
- * separately (FP64 with no x-sweep tile
+ * separately (by strips in LDS where rows fit; otherwise FP64 with no x-sweep tile
  * of more than 3072 occupied voxels: one fused launch; otherwise phases 0 and 1); enqueued
  * `count` times on the context's stream. */
 int bfvmb_launch_phase(bfvmb_ctx *ctx, int phase, int count);

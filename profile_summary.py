@@ -64,14 +64,15 @@ def traffic(fetch_db, write_db, out):
         cal[label] = COPY_BYTES / big if big else 1.0
     res, rows = {}, []
     # k_sweep_x<T, PC, REGC, TL, VF, AG[, NT]>: AG = the step's agent update in the same launch
-    phase = {"k_sweep_x": "sweep_x", "k_sweep_yz<double, 1": "sweep_y", "k_sweep_yz<double, 2": "sweep_z"}
+    # k_strip<T, AG, NT>: the same, by strips in LDS
+    phase = {"k_sweep_x": "sweep_x", "k_strip": "sweep_x", "k_sweep_yz<double, 1": "sweep_y", "k_sweep_yz<double, 2": "sweep_z"}
 
     def template_args(name):
         return name[name.index("<") + 1:name.rindex(">")].split(", ") if "<" in name else []
 
     for k in f:
         s = short(k)
-        if "k_sweep" not in s and "k_agents" not in s:
+        if "k_sweep" not in s and "k_strip" not in s and "k_agents" not in s:
             continue
         fb = sum(f[k]) / len(f[k]) * cal["fetch"]
         wb = sum(w.get(k, [0.0])) / max(1, len(w.get(k, [0.0]))) * cal["write"]
@@ -79,22 +80,23 @@ def traffic(fetch_db, write_db, out):
         for pre, ph in phase.items():
             if s.startswith(pre) and "double" in s:
                 args = template_args(s)
-                if ph == "sweep_x" and len(args) >= 6 and args[5] == "true":
+                if ph == "sweep_x" and (args[1] == "true" if pre == "k_strip" else len(args) >= 6 and args[5] == "true"):
                     ph = "sweep_x_with_agents"
                 res[ph] = fb + wb
-    # provenance: the sweep source these counters describe (bench.py reports the traffic only
-    # while biofvm-b_amd/csrc/lod.hip still has this hash) and the commit checked out
+    # provenance: the sweep sources these counters describe (bench.py reports the traffic only
+    # while lod.hip and resident.hip in biofvm-b_amd/csrc still have this hash) and the commit
     import hashlib
     import os
     import subprocess
     root = os.path.dirname(os.path.abspath(__file__))
-    sha = hashlib.sha256(open(os.path.join(root, "biofvm-b_amd", "csrc", "lod.hip"), "rb").read()).hexdigest()
+    sha = hashlib.sha256(b"".join(open(os.path.join(root, "biofvm-b_amd", "csrc", f), "rb").read()
+                                  for f in ("lod.hip", "resident.hip"))).hexdigest()
     try:
         commit = subprocess.run(["git", "-C", root, "rev-parse", "--short=12", "HEAD"], capture_output=True,
                                 text=True, check=True).stdout.strip()
     except (OSError, subprocess.CalledProcessError):
         commit = None
-    json.dump({"bytes_per_launch": res, "calibration": cal, "lod_hip_sha256": sha, "commit": commit},
+    json.dump({"bytes_per_launch": res, "calibration": cal, "sweep_source_sha256": sha, "commit": commit},
               open(out, "w"), indent=1)
     print(f"calibration (true bytes / counter bytes of the 1 GiB copy): fetch {cal['fetch']:.3f}, write {cal['write']:.3f}")
     print("| kernel | fetched (GB/launch) | written (GB/launch) | total (GB) |")
